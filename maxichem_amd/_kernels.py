@@ -94,6 +94,42 @@ def words_in_lds(tab: Tables, cpw: int, mixed: bool = False, wps: int = 1, rates
     return words <= CU_LDS and per_cu(words) >= per_cu(cells)
 
 
+# The two-dimensional LU up to here: its block takes 180 registers at 69 species and 276 at 92, which a wavefront alone
+# on its SIMD holds (256, and accumulation registers for what rests); 128 species would take 512. Larger networks keep
+# the LU by rows.
+LU_MAX_SPECIES = 92
+
+
+def lu_layout(tab: Tables) -> dict:
+    """The two-dimensional LU's layout (kernels/common.hip, factor_2d): register slots of 16 rows (m) by 4 columns
+    (t), the lead rows' and columns' (ml, tl) first; per pivot, the row slots that hold an entry below it in its column
+    and the column slots that hold one right of it in its row, in the filled pattern; per row slot, the column slots
+    that hold any entry. The trailing rows' columns pass through the cell's LDS from its dv terms to its trash slots,
+    chunk column slots of stride doubles a column at a time."""
+    ns, k0, nt, fill, lay = tab.ns, tab.k0, tab.nt, tab.fill, tab.layout()
+    ml, tl = -(-k0 // 16), -(-k0 // 4)
+    m, t = ml + -(-nt // 16), tl + -(-nt // 4)
+    row = np.array([i // 16 if i < k0 else ml + (i - k0) // 16 for i in range(ns)])
+    col = np.array([j // 4 if j < k0 else tl + (j - k0) // 4 for j in range(ns)])
+
+    def bits(slots) -> int:
+        return sum(1 << int(q) for q in np.unique(slots))
+
+    rows = [bits(row[np.flatnonzero(fill[k + 1 :, k]) + k + 1]) for k in range(ns)]
+    cols = [bits(col[np.flatnonzero(fill[k, k + 1 :]) + k + 1]) for k in range(ns)]
+    live = [bits(col[np.flatnonzero(fill[row == r].any(0))]) for r in range(m)]
+    room = lay["TRASH"] + C.WAVE - lay["DV"]
+    stride = 16 * (m - ml)
+    # 16 doubles more a column put neighbouring columns on other banks, where that costs no more chunks
+    plain, wide = (min(t, room // (4 * q)) for q in (stride, stride + 16))
+    if wide and -(-t // wide) == -(-t // plain):
+        stride, plain = stride + 16, wide
+    need = max(64 * m, 16 * m + 4 * tl + C.WAVE)  # the multipliers' exchange; the diagonal and its reciprocals
+    fits = plain > 0 and room >= need and 16 * ml * ns <= lay["TRASH"] + C.WAVE  # whole slots of lead rows are read
+    return {"use": ns <= LU_MAX_SPECIES and fits, "m": m, "t": t, "ml": ml, "tl": tl,
+            "rows": rows, "cols": cols, "live": live, "chunk": max(plain, 1), "stride": stride}  # fmt: skip
+
+
 def header(tab: Tables, cpw: int, drift: float, batch: int = DEFAULT_BATCH, mixed: bool = False, wps: int = 1,
            rates_global: bool = False, words_lds: bool = False) -> str:
     """The network header: every size, offset and setting the kernel files read. cpw: cells (wavefronts) per
@@ -132,6 +168,8 @@ def header(tab: Tables, cpw: int, drift: float, batch: int = DEFAULT_BATCH, mixe
     jp = jv + 4 * (tab.nr + 1)
     jsize = jp + 4 * tab.npart
     ints.update({"J_KD": 0, "J_N": jn, "J_G": jn, "J_V": jv, "J_PART": jp, "J_SIZE": jsize + (jsize & 1)})
+    lu = lu_layout(tab)
+    ints.update({"LU_M": lu["m"], "LU_T": lu["t"], "LU_ML": lu["ml"], "LU_TL": lu["tl"], "LU_CHUNK": lu["chunk"], "LU_STRIDE": lu["stride"]})
     lines = [f"// network header: {tab.ns} species, {tab.nr} reactions, tables {tab.digest()}"]
     lines += [f"constexpr int {k} = {v};" for k, v in ints.items()]
     lines += [f"constexpr double {k} = {v!r};" for k, v in doubles.items()]
@@ -145,6 +183,9 @@ def header(tab: Tables, cpw: int, drift: float, batch: int = DEFAULT_BATCH, mixe
         # the trailing rows' filled pattern: bit j of TRAIL_FILL[t] is column K0 + j of row K0 + t
         f"__device__ constexpr unsigned long long TRAIL_FILL[{tab.nt}] = "
         f"{{{', '.join(f'{m}ull' for m in tab.trail_fill)}}};",
+        f"constexpr bool LU_2D = {'true' if lu['use'] else 'false'};",
+        *(f"__device__ constexpr unsigned {name}[{len(lu[key])}] = {{{', '.join(f'{v}u' for v in lu[key])}}};"
+          for name, key in (("LU_ROWS", "rows"), ("LU_COLS", "cols"), ("LU_LIVE", "live"))),
         f"#define HAS_TROE {int(tab.has_troe)}",
         f"#define MIXED {int(mixed)}",
         f"#define CALL_WAVES_PER_SIMD {int(wps)}",

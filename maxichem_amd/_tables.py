@@ -159,6 +159,7 @@ class Tables:
     sv_words: np.ndarray = field(default=None)  # uint32 [rounds, 64]
     npart: int = 0
     row_pieces: np.ndarray = field(default=None)  # uint32 [ns]: first piece | count << 16
+    fill: np.ndarray = field(default=None)  # bool [ns, ns]: the unpivoted LU's filled pattern, elimination order
     jac_terms: int = 0
     sv_terms: int = 0
     live: int = 0
@@ -278,6 +279,7 @@ def build(net: VulcanNetwork, photo: bool = False) -> Tables:
     )  # fmt: skip
     tab.ndv, tab.live = ndv, len(live)
     tab.trail_fill = trail_fill
+    tab.fill = fill
     if ndv >= (1 << T_IDX_BITS) - 1 or nr >= (1 << SV_R_BITS):
         raise ValueError(f"the network is too large for the kernel's streams: {ndv} derivative terms, {nr} reactions")
     # reaction words: species in elimination order (pad ns), dv offset

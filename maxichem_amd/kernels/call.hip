@@ -52,11 +52,17 @@ __device__ __forceinline__ bool stages(T (&c)[NT], LeadRow& a21, double Nl, doub
   const double igh = 1.0 / (GAMMA * ha), ih = 1.0 / ha;
   double Fl = 0.0, Ft = 0.0, ul = 0.0, ut = 0.0, u0l = 0.0, u0t = 0.0;
   const double ntot = rhs<true, WORDS_LDS != 0>(Nl, Nt, Fl, Ft, u0l, u0t, net, nd, ws, rk, lane);
-  jacobian<WORDS_LDS != 0>(c, a21, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
-  add_diagonal(c, igh, ws, lane);
   double dl;
   T dtr;
-  factor_m0(c, a21, dl, dtr, ws, lane);
+  if constexpr (LU_2D && sizeof(T) == sizeof(double)) {
+    LuBlock A;
+    lu_assemble<WORDS_LDS != 0>(A, igh, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
+    lu_factor(A, c, a21, dl, dtr, ws, lane);
+  } else {
+    jacobian<WORDS_LDS != 0>(c, a21, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
+    add_diagonal(c, igh, ws, lane);
+    factor_m0(c, a21, dl, dtr, ws, lane);
+  }
   const double wl = atol + rtol * fabs(Nl), wt = atol + rtol * fabs(Nt);  // the refinement's error weights
 #define MXC_SOLVE(YL, YT) \
   if (!solve_m0(YL, YT, c, a21, dl, dtr, igh, wl, wt, net, ws, lane)) return false
@@ -105,7 +111,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW) __attribute__((amdgpu_wa
              double rtol, double atol, int max_steps, const double* __restrict__ xprop,
              double* __restrict__ rscratch, int* __restrict__ fp64) {
   extern __shared__ double lds[];
-  const int lane = (int)(threadIdx.x & (WAVE - 1)), wv = (int)(threadIdx.x / WAVE);
+  // the wavefront's index as a scalar: its cell, and so the loops over cells and tries, are then known to be uniform
+  const int lane = (int)(threadIdx.x & (WAVE - 1)), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
   double* ws = lds + wv * L_SIZE;
 #if RATES_GLOBAL
   double* rk = rscratch + (size_t)((int)blockIdx.x * CPW + wv) * (2 * NR);  // this wave's slot

@@ -113,14 +113,21 @@ __device__ __forceinline__ int wave_min(int v) {
 // computed there and not all ahead of the loop, where they would fill the scalar registers.
 __device__ __forceinline__ int opaque_lane(int lane) {
   asm volatile("" : "+v"(lane));
-  return lane;
+  return lane & (WAVE - 1);  // known to be a lane: a test of it against a whole wavefront's rows folds
+}
+
+// The cell's LDS region as an opaque place, for the same reason: its addresses made where they are used.
+__device__ __forceinline__ double* opaque_lds(double* ws) {
+  int zero = 0;
+  asm volatile("" : "+s"(zero));
+  return ws + zero;
 }
 
 // The lane index as an opaque value that the compiler must take after x is computed: a step's lane mask then
 // cannot be computed ahead of the step whose value x it follows.
 __device__ __forceinline__ int lane_after(int lane, double x) {
   asm volatile("" : "+v"(lane) : "v"(x));
-  return lane;
+  return lane & (WAVE - 1);
 }
 
 // The table pointer p, made opaque to the compiler where it is used, so that the loads and decodes from the
@@ -237,6 +244,8 @@ __device__ __forceinline__ int species_of(u64 w, int m) { return (int)((w >> (8 
 // collision limit, a photolysis branch's kf = J exp(lm) (the reference's tangent kernels' rates, ad_common.cuh:136-168)
 __device__ __forceinline__ void cell_rates(double* ws, double* rk, double T, double nd, NetP net,
                                            const double* Jc, int lane, const double* lmc = nullptr) {
+  ws = opaque_lds(ws);
+  lane = opaque_lane(lane);
   net = opaque(net);
   const gptr<double> rc = net->rc;
   const gptr<int> rf = net->rf;
@@ -357,6 +366,8 @@ __device__ __forceinline__ const u32* lds_words(const double* ws) {  // ws: this
 template <bool JAC, bool LW = false>
 __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& Ft, double& u0l, double& u0t,
                                       NetP net, double nd, double* ws, const double* rk, int lane) {
+  ws = opaque_lds(ws);
+  lane = opaque_lane(lane);
   const double ntot = wave_sum((lane < K0 ? Yl : 0.0) + (lane < NT ? Yt : 0.0));
   const double xf = nd / ntot, ixf = ntot / nd;
   double* n = ws + L_NVEC;
@@ -437,12 +448,65 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
   return ntot;
 }
 
-// -Jn into LEAD (LDS), the trailing rows' lead columns a21 and the trailing block c (registers), from the dv terms
-// that rhs<true> left in DV; then u = w = S v / nd - Jn N / n_tot, the constant-pressure part of the exact Jacobian
-// (lead / trailing parts).
-template <bool LW = false, typename T>
-__device__ __forceinline__ void jacobian(T (&c)[NT], LeadRow& a21, double Nl, double Nt, double u0l, double u0t,
-                                         double ntot, double& ul, double& ut, NetP net, double* ws, int lane) {
+// ---- -Jn from the dv terms that rhs<true> left in DV ----
+
+template <int... K>
+struct Seq {};
+template <typename T, T... K>
+struct IntSeq : Seq<K...> {};
+template <int N>
+using Steps = __make_integer_seq<IntSeq, int, N>;
+
+// One chunk of CHUNK columns of the trailing rows' -Jn, through the staging area (column-major) into sink.chunk, and
+// its part of -Jn N. Chunks 0 .. NLCH - 1 hold the lead columns (K0 > 0 means NT == WAVE: every lane has a trailing
+// row), the others the trailing columns. cd: the row's own diagonal entry, which the chunk streams do not hold.
+template <bool LW, int CH, typename Sink>
+__device__ __forceinline__ void jac_chunk(Sink& sink, double cd, double Nl, double Nt, double& mt, const double* xv,
+                                          NetP net, double* ws, int lane) {
+  const double* DV = ws + L_DV;
+  double* stage = ws + L_STAGE;
+  constexpr int C0 = (CH < NLCH ? CH : CH - NLCH) * CHUNK, NC = CH < NLCH ? K0 : NT;  // its first column, of NC
+  if (lane < NT) {
+#pragma unroll
+    for (int j = 0; j < CHUNK; j++) stage[j * NT + lane] = 0.0;
+    if (CH >= NLCH && lane / CHUNK == CH - NLCH) stage[(lane % CHUNK) * NT + lane] = cd;
+  }
+  wave_sync();
+  if constexpr (LW)
+    jac_stream(lds_words(ws) + W_CH + CH_OFF[CH] * WAVE, CH_ROUNDS[CH], DV, ws, lane);
+  else
+    jac_stream(opaque(net)->chw + CH_OFF[CH] * WAVE, CH_ROUNDS[CH], DV, ws, lane);
+  wave_sync();
+  // N_j for -Jn N as wave-uniform values: with few lead rows from the exchange vector (same-address LDS reads, kept in
+  // their chunk: hoisted ahead, they would hold a register pair each), else by v_readlane
+  double nj[CHUNK], v[CHUNK];
+  if constexpr (K0 <= SMALL_LEAD) {
+#pragma unroll
+    for (int j = 0; j < CHUNK; j++) nj[j] = xv[(CH < NLCH ? 0 : K0) + (C0 + j < NC ? C0 + j : 0)];
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int j = 0; j < CHUNK; j++) v[j] = C0 + j < NC && lane < NT ? stage[j * NT + lane] : 0.0;
+  sink.template chunk<CH>(v, stage, lane);
+#pragma unroll
+  for (int j = 0; j < CHUNK; j++)
+    if (C0 + j < NC) mt = fma(v[j], K0 <= SMALL_LEAD ? nj[j] : readlane(CH < NLCH ? Nl : Nt, C0 + j), mt);
+  pin(mt);  // taken here: left to its use after the factorization, the chunk's entries would be held until then
+}
+
+template <bool LW, typename Sink, int... CH>
+__device__ __forceinline__ void jac_chunks(Seq<CH...>, Sink& sink, double cd, double Nl, double Nt, double& mt,
+                                           const double* xv, NetP net, double* ws, int lane) {
+  (jac_chunk<LW, CH>(sink, cd, Nl, Nt, mt, xv, net, ws, lane), ...);
+}
+
+// -Jn: the lead rows into LEAD (LDS), the trailing rows to sink, from the dv terms in DV; then u = w = S v / nd -
+// Jn N / n_tot, the constant-pressure part of the exact Jacobian (lead / trailing parts).
+template <bool LW, typename Sink>
+__device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, double u0l, double u0t, double ntot,
+                                             double& ul, double& ut, NetP net, double* ws, int lane) {
+  lane = opaque_lane(lane);
+  ws = opaque_lds(ws);
   double* DV = ws + L_DV;
   for (int s = lane; s < L_NVEC; s += WAVE) ws[s] = 0.0;  // LEAD
   if (lane < NT) ws[L_DIAG + lane] = 0.0;                   // a species in no reaction has no diagonal term
@@ -460,12 +524,11 @@ __device__ __forceinline__ void jacobian(T (&c)[NT], LeadRow& a21, double Nl, do
     jac_stream(opaque(net)->leadw, LEAD_ROUNDS, DV, ws, lane);
   }
   wave_sync();
-  // -Jn N in FP64, from the entries before the trailing block takes them in T: the lead rows through the exchange
-  // vector, then the trailing rows chunk by chunk (their lead columns, then the trailing ones), N_j from lane j
+  // -Jn N in FP64: the lead rows through the exchange vector, then the trailing rows chunk by chunk (their lead
+  // columns, then the trailing ones)
   double ml = 0.0, mt = 0.0;
   if constexpr (K0 > 0 && K0 <= SMALL_LEAD) {
-    // few lead rows: each row times N as this lane's share (its own N entries), summed over the lanes; the trailing
-    // rows' lead columns times N with N_k by v_readlane
+    // few lead rows: each row times N as this lane's share (its own N entries), summed over the lanes
     double sum[K0 > 0 ? K0 : 1];
 #pragma unroll
     for (int i = 0; i < K0; i++)
@@ -488,52 +551,33 @@ __device__ __forceinline__ void jacobian(T (&c)[NT], LeadRow& a21, double Nl, do
     }
   }
   const double cd = lane < NT ? ws[L_DIAG + lane] : 0.0;
-  double* stage = ws + L_STAGE;
-  // chunks 0 .. NLCH - 1 hold the lead columns (K0 > 0 means NT == WAVE: every lane has a trailing row), the
-  // others the trailing columns from t0
-#pragma unroll
-  for (int ch = 0; ch < NCH; ch++) {
-    const int t0 = (ch - NLCH) * CHUNK;
-    if (lane < NT) {
-#pragma unroll
-      for (int j = 0; j < CHUNK; j++) stage[j * NT + lane] = 0.0;
-      // the chunk streams hold no diagonal entry: a trailing row's own diagonal goes in by its lane
-      if (ch >= NLCH && lane / CHUNK == ch - NLCH) stage[(lane % CHUNK) * NT + lane] = cd;
-    }
-    wave_sync();
-    if constexpr (LW)
-      jac_stream(lds_words(ws) + W_CH + CH_OFF[ch] * WAVE, CH_ROUNDS[ch], DV, ws, lane);
-    else
-      jac_stream(opaque(net)->chw + CH_OFF[ch] * WAVE, CH_ROUNDS[ch], DV, ws, lane);
-    wave_sync();
-    // N_j for -Jn N as wave-uniform values: with few lead rows from the exchange vector (same-address LDS reads,
-    // kept in their chunk: hoisted ahead, they would hold a register pair each), else by v_readlane (with the lead
-    // columns in registers the LDS reads' registers make the kernel spill)
-    double nj[CHUNK];
-    if constexpr (K0 <= SMALL_LEAD) {
-#pragma unroll
-      for (int j = 0; j < CHUNK; j++)
-        nj[j] = ch < NLCH ? xv[ch * CHUNK + j < K0 ? ch * CHUNK + j : 0] : xv[K0 + (t0 + j < NT ? t0 + j : 0)];
-      asm volatile("" ::: "memory");
-    }
-#pragma unroll
-    for (int j = 0; j < CHUNK; j++) {
-      if (ch < NLCH) {
-        if (ch * CHUNK + j < K0) {
-          const double v = stage[j * NT + lane];
-          a21[ch * CHUNK + j] = v;
-          mt = fma(v, K0 <= SMALL_LEAD ? nj[j] : readlane(Nl, ch * CHUNK + j), mt);
-        }
-      } else if (t0 + j < NT) {
-        const double v = lane < NT ? stage[j * NT + lane] : 0.0;
-        c[t0 + j] = (T)v;
-        mt = fma(v, K0 <= SMALL_LEAD ? nj[j] : readlane(Nt, t0 + j), mt);
-      }
-    }
-  }
+  jac_chunks<LW>(Steps<NCH>{}, sink, cd, Nl, Nt, mt, xv, net, ws, lane);
   ul = u0l + ml / ntot;
   ut = lane < NT ? u0t + mt / ntot : 0.0;
   wave_sync();
+}
+
+// The trailing rows by lane: their lead columns into a21, the trailing block into c.
+template <typename T>
+struct RowSink {
+  T (&c)[NT];
+  LeadRow& a21;
+  template <int CH>
+  __device__ __forceinline__ void chunk(const double (&v)[CHUNK], const double*, int) {
+#pragma unroll
+    for (int j = 0; j < CHUNK; j++) {
+      if (CH < NLCH && CH * CHUNK + j < K0) a21[CH * CHUNK + j < K0 ? CH * CHUNK + j : 0] = v[j];
+      if (CH >= NLCH && (CH - NLCH) * CHUNK + j < NT) c[(CH - NLCH) * CHUNK + j < NT ? (CH - NLCH) * CHUNK + j : 0] = (T)v[j];
+    }
+  }
+};
+
+// -Jn by rows: LEAD (LDS), the trailing rows' lead columns a21 and the trailing block c (registers).
+template <bool LW = false, typename T>
+__device__ __forceinline__ void jacobian(T (&c)[NT], LeadRow& a21, double Nl, double Nt, double u0l, double u0t,
+                                         double ntot, double& ul, double& ut, NetP net, double* ws, int lane) {
+  RowSink<T> sink{c, a21};
+  jac_assemble<LW>(sink, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
 }
 
 // ---- the unpivoted LU of M0 in the elimination order, and its solves ----
@@ -541,6 +585,8 @@ __device__ __forceinline__ void jacobian(T (&c)[NT], LeadRow& a21, double Nl, do
 // Adds 1 / (gamma h) to M0's diagonal: the lead rows in LDS, the trailing block in registers.
 template <typename T>
 __device__ __forceinline__ void add_diagonal(T (&c)[NT], double igh, double* ws, int lane) {
+  ws = opaque_lds(ws);
+  lane = opaque_lane(lane);
   if (lane < K0) ws[lane * NS + lane] += igh;
 #pragma unroll
   for (int j = 0; j < NT; j++) c[j] += j == lane ? (T)igh : (T)0;
@@ -665,11 +711,301 @@ __device__ __forceinline__ void factor_trailing(double (&c)[NT], double& dt, dou
   wave_sync();
 }
 
-// LU of the lead columns (right-looking, dense in LDS), the Schur update of the trailing block, then the trailing
-// block's LU in registers. dl: 1 / U_ii of lead row lane; dt: of trailing row lane.
-__device__ __forceinline__ void factor(double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws, int lane) {
+// ---- the LU of the whole of M0 in registers, 16 rows by 4 columns to a register ----
+//
+// Lane (g, s) = (lane / 16, lane % 16) holds A[m][t], the entry of row s of row slot m and column g of column slot t:
+// slots of the lead rows (LU_ML) and columns (LU_TL) first, then of the trailing ones. A pivot's row then sits in one
+// lane of each row of 16 lanes, and the updates take it by one DPP row broadcast for all of a lane's rows; a pivot's
+// column sits in the 16 lanes of one g, and its multipliers reach the others through LDS, a write and a read per 16
+// rows. Each entry takes its updates pivot by pivot, so the factors have the same bits in every layout. Slots that the
+// filled pattern keeps zero (LU_ROWS, LU_COLS, LU_LIVE) are left out.
+//
+// What bounds it is the issue of one wavefront's instructions. By rows (factor_rows) an update costs an fma and the two
+// v_readlane of its broadcast; here a broadcast (v_mov_b64_dpp) serves the 16 rows of up to LU_M slots, and a pivot's
+// chain (broadcast, reciprocal, LDS round trip) runs beside the previous pivot's updates. Cycles of one wavefront per
+// factorization, the lead rows' LU and Schur update included: NCHO (69 species) 40.3k by rows, 24k here; SNCHO (91,
+// 27 lead rows, whose LU by rows goes through LDS) 183k and 41k.
+typedef double LuBlock[LU_M][LU_T];
+
+// v of lane K of each row of 16 lanes, in the row's lanes; with ROWS only in those rows of lanes, 0 in the others.
+template <int K, int ROWS = 0xf>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __longlong_as_double(
+      __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + K, ROWS, 0xf, ROWS == 0xf));
+}
+
+// 1 / x without the division's scaling steps, which change nothing while x and 1 / x are normal numbers: the same two
+// Newton steps and final correction on v_rcp_f64, and the same fixup of zeros, infinities and NaN.
+__device__ __forceinline__ double plain_rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return __builtin_amdgcn_div_fixup(fma(fma(-x, r, 1.0), r, r), x, 1.0);
+}
+
+// Pivot K's place: its row slot and row, its column slot and column.
+template <int K>
+struct Pivot {
+  static constexpr int R = K < K0 ? K : K - K0;
+  static constexpr int M = (K < K0 ? 0 : LU_ML) + R / 16, S = R % 16, T = (K < K0 ? 0 : LU_TL) + R / 4, G = R % 4;
+};
+
+// Pivot K's multipliers -l_i K of this lane's rows (0 up to row K) from its column; lb: their exchange, [4][16 LU_M] in
+// LDS (each row of lanes writes its own part, the pivot's is read). The column itself keeps its unscaled entries.
+template <int K>
+__device__ __forceinline__ void lu_pivot(const LuBlock& A, double (&nl)[LU_M], double* lb, int lane) {
+  using P = Pivot<K>;
+  const double dk = plain_rcp(readlane(A[P::M][P::T], 16 * P::G + P::S));
+  const int s = opaque_lane(lane & 15);  // the step's mask made here
+  double* mine = lb + (lane >> 4) * (16 * LU_M) + (lane & 15);
+#pragma unroll
+  for (int m = P::M; m < LU_M; m++)
+    if ((LU_ROWS[K] >> m) & 1u) {
+      const double x = A[m][P::T] * dk;
+      mine[16 * m] = m > P::M || s > P::S ? x : 0.0;
+    }
+  wave_sync();
+#pragma unroll
+  for (int m = P::M; m < LU_M; m++)
+    if ((LU_ROWS[K] >> m) & 1u) nl[m] = -lb[P::G * (16 * LU_M) + 16 * m + (lane & 15)];
+  wave_sync();
+}
+
+// Pivot K's update of column slot t.
+template <int K>
+__device__ __forceinline__ void lu_update(LuBlock& A, const double (&nl)[LU_M], int t) {
+  using P = Pivot<K>;
+  if (!((LU_COLS[K] >> t) & 1u)) return;
+  const double u =
+      t > P::T ? row_bcast<P::S>(A[P::M][t]) : row_bcast<P::S, (0xf << (P::G + 1)) & 0xf>(A[P::M][t]);
+#pragma unroll
+  for (int m = P::M; m < LU_M; m++)
+    if ((LU_ROWS[K] >> m) & 1u) A[m][t] = fma(nl[m], u, A[m][t]);
+}
+
+// Pivot K's updates, with pivot K + 1's multipliers (a chain of a broadcast, a reciprocal and an LDS round trip) taken
+// as soon as its own column is final, while the other columns are updated.
+template <int K>
+__device__ __forceinline__ void lu_step(LuBlock& A, double (&nl)[LU_M], double* lb, int lane) {
+  __builtin_amdgcn_sched_barrier(0);
+  constexpr int TN = Pivot<K + 1 < NS ? K + 1 : K>::T;
+  double next[LU_M];
+  if constexpr (K + 1 < NS) {
+    lu_update<K>(A, nl, TN);
+    lu_pivot<K + 1>(A, next, lb, lane);
+  }
+#pragma unroll
+  for (int t = Pivot<K>::T; t < LU_T; t++)
+    if (t != TN) lu_update<K>(A, nl, t);
+  if constexpr (K + 1 < NS) {
+#pragma unroll
+    for (int m = 0; m < LU_M; m++) nl[m] = next[m];
+  }
+}
+
+template <int... K>
+__device__ __forceinline__ void lu_steps(Seq<K...>, LuBlock& A, double* lb, int lane) {
+  double nl[LU_M];
+  lu_pivot<0>(A, nl, lb, lane);
+  (lu_step<K>(A, nl, lb, lane), ...);
+}
+
+// A lane's place of slot (m, t) in a chunk of columns, column-major with LU_STRIDE doubles a column for the trailing
+// rows' slots, or in the lead rows.
+struct LuPlace {
+  double *chunk, *lead;
+  __device__ __forceinline__ LuPlace(double* ws, int lane)
+      : chunk(ws + L_DV + (lane >> 4) * LU_STRIDE + (lane & 15)), lead(ws + (lane & 15) * NS + (lane >> 4)) {}
+  __device__ __forceinline__ double* at(int m, int t, int t0) const {
+    return m < LU_ML ? lead + 16 * m * NS + (t < LU_TL ? 4 * t : K0 + 4 * (t - LU_TL))
+                     : chunk + 4 * (t - t0) * LU_STRIDE + 16 * (m - LU_ML);
+  }
+};
+
+// Whether this lane's entry of slot (m, t) is inside the matrix (the slots' last rows and columns may not be).
+__device__ __forceinline__ bool lu_inside(int m, int t, int lane) {
+  const int i = m < LU_ML ? 16 * m : 16 * (m - LU_ML), j = t < LU_TL ? 4 * t : 4 * (t - LU_TL);
+  const int ni = m < LU_ML ? K0 : NT, nj = t < LU_TL ? K0 : NT;
+  return (i + 16 <= ni || i + (lane & 15) < ni) && (j + 4 <= nj || j + (lane >> 4) < nj);
+}
+
+// A from the rows by lane (c, a21, and the lead rows in LDS; a caller that has the matrix by rows): columns pass LU_CHUNK slots at a time through the cell's
+// LDS from its dv terms on, which no later part of a try reads.
+__device__ __forceinline__ void lu_load(LuBlock& A, const double (&c)[NT], const LeadRow& a21, double* ws, int lane) {
+  const LuPlace p(ws, lane);
+  double* buf = ws + L_DV;
+#pragma unroll
+  for (int t0 = 0; t0 < LU_T; t0 += LU_CHUNK) {
+    if (lane < NT) {
+#pragma unroll
+      for (int t = t0; t < t0 + LU_CHUNK && t < LU_T; t++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const int j = t < LU_TL ? 4 * t + g : 4 * (t - LU_TL) + g;
+          if (t < LU_TL ? j < K0 : j < NT)
+            buf[(4 * (t - t0) + g) * LU_STRIDE + lane] = t < LU_TL ? a21[j < K0 ? j : 0] : c[j < NT ? j : 0];
+        }
+    }
+    wave_sync();
+#pragma unroll
+    for (int m = 0; m < LU_M; m++)
+#pragma unroll
+      for (int t = t0; t < t0 + LU_CHUNK && t < LU_T; t++) {
+        A[m][t] = 0.0;
+        if ((LU_LIVE[m] >> t) & 1u) {
+          const double v = *p.at(m, t, t0);  // outside the matrix: some place of the cell's
+          A[m][t] = lu_inside(m, t, lane) ? v : 0.0;
+        }
+      }
+    wave_sync();
+  }
+}
+
+// The factors out of A: 1 / U_ii of lead row lane (dl) and of trailing row lane (dt); each column times its 1 / U_jj
+// below the diagonal (L) and, in the trailing rows, above it (U' = U diag(1 / U_jj)); and the rows back to their lanes.
+__device__ __forceinline__ void lu_store(LuBlock& A, double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
+                                         int lane) {
+  const LuPlace p(ws, lane);
+  const int s = lane & 15, g = lane >> 4, q = s >> 2;
+  double* buf = ws + L_DV;
+  // the diagonal: row s of a row slot has it in column slot s / 4 of the slot's four, in the lanes of g = s % 4
+  double dg[LU_M];
+#pragma unroll
+  for (int m = 0; m < LU_M; m++) {
+    const int t0 = m < LU_ML ? 4 * m : LU_TL + 4 * (m - LU_ML), last = m < LU_ML ? LU_TL : LU_T;
+    dg[m] = A[m][t0];
+#pragma unroll
+    for (int u = 1; u < 4; u++)
+      if (t0 + u < last) dg[m] = q == u ? A[m][t0 + u] : dg[m];
+  }
+  if (g == (s & 3)) {
+#pragma unroll
+    for (int m = 0; m < LU_M; m++) buf[16 * m + s] = dg[m];
+  }
+  wave_sync();
+  double* dinv = buf + 16 * LU_M;  // by column, a slot's four together
+  dl = lane < K0 ? 1.0 / buf[lane < K0 ? lane : 0] : 1.0;
+  dt = lane < NT ? 1.0 / buf[16 * LU_ML + lane] : 1.0;
+  if (lane < 4 * LU_TL) dinv[lane] = dl;
+  dinv[4 * LU_TL + lane] = dt;
+  wave_sync();
+#pragma unroll
+  for (int t = 0; t < LU_T; t++) {
+    const double d = dinv[4 * t + g];
+#pragma unroll
+    for (int m = 0; m < LU_M; m++) {
+      const bool lead_u = m < LU_ML && (t >= LU_TL || t / 4 > m);  // a lead row's slot right of its diagonal
+      if (!((LU_LIVE[m] >> t) & 1u) || lead_u) continue;
+      const bool diag = m < LU_ML ? t < LU_TL && t / 4 == m : t >= LU_TL && (t - LU_TL) / 4 == m - LU_ML;
+      const int j = 4 * (m < LU_ML ? t & 3 : (t - LU_TL) & 3) + g;  // the column's row in a diagonal slot
+      A[m][t] *= !diag || s > j || (m >= LU_ML && s != j) ? d : 1.0;
+    }
+  }
+  wave_sync();
+#pragma unroll
+  for (int t0 = 0; t0 < LU_T; t0 += LU_CHUNK) {
+#pragma unroll
+    for (int m = 0; m < LU_M; m++)
+#pragma unroll
+      for (int t = t0; t < t0 + LU_CHUNK && t < LU_T; t++)
+        if (m >= LU_ML || (((LU_LIVE[m] >> t) & 1u) && lu_inside(m, t, lane))) *p.at(m, t, t0) = A[m][t];
+    wave_sync();
+    if (lane < NT) {
+#pragma unroll
+      for (int t = t0; t < t0 + LU_CHUNK && t < LU_T; t++)
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+          const int j = t < LU_TL ? 4 * t + h : 4 * (t - LU_TL) + h;
+          const double v = buf[(4 * (t - t0) + h) * LU_STRIDE + lane];
+          if (t < LU_TL) {
+            if (j < K0) a21[j < K0 ? j : 0] = v;
+          } else if (j < NT) {
+            c[j < NT ? j : 0] = v;
+          }
+        }
+    }
+    wave_sync();
+  }
+}
+
+// The trailing rows' slots, from the staging area.
+struct LuSink {
+  LuBlock& A;
+  template <int CH>
+  __device__ __forceinline__ void chunk(const double (&)[CHUNK], const double* stage, int lane) {
+    constexpr int T0 = CH < NLCH ? CH * (CHUNK / 4) : LU_TL + (CH - NLCH) * (CHUNK / 4), END = CH < NLCH ? LU_TL : LU_T;
+    const double* p = stage + (lane >> 4) * NT + (lane & 15);
+#pragma unroll
+    for (int t = T0; t < T0 + CHUNK / 4 && t < END; t++)
+#pragma unroll
+      for (int m = LU_ML; m < LU_M; m++) {
+        A[m][t] = 0.0;
+        if ((LU_LIVE[m] >> t) & 1u) {
+          const double v = p[4 * (t - T0) * NT + 16 * (m - LU_ML)];  // outside the matrix: some place of the cell's
+          A[m][t] = lu_inside(m, t, lane) ? v : 0.0;
+        }
+      }
+  }
+};
+
+// M0 = igh - Jn into A's slots, LEAD, and u as jacobian's.
+template <bool LW>
+__device__ __forceinline__ void lu_assemble(LuBlock& A, double igh, double Nl, double Nt, double u0l, double u0t,
+                                            double ntot, double& ul, double& ut, NetP net, double* ws, int lane) {
+  LuSink sink{A};
+  jac_assemble<LW>(sink, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
+  lane = opaque_lane(lane);
+  const LuPlace p(opaque_lds(ws), lane);
+  const int s = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < LU_ML; m++)
+#pragma unroll
+    for (int t = 0; t < LU_T; t++) {
+      A[m][t] = 0.0;
+      if ((LU_LIVE[m] >> t) & 1u) {
+        const double v = *p.at(m, t, 0);
+        A[m][t] = lu_inside(m, t, lane) ? v : 0.0;
+      }
+    }
+#pragma unroll
+  for (int m = 0; m < LU_M; m++) {
+    const int t0 = m < LU_ML ? 4 * m : LU_TL + 4 * (m - LU_ML), last = m < LU_ML ? LU_TL : LU_T;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (t0 + u < last) A[m][t0 + u] += s == 4 * u + g ? igh : 0.0;
+  }
+  wave_sync();
+}
+
+// The LU of A into the rows by lane, and the reciprocals of its diagonal.
+__device__ __forceinline__ void lu_factor(LuBlock& A, double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
+                                          int lane) {
+  lane = opaque_lane(lane);
+  ws = opaque_lds(ws);
+  lu_steps(Steps<NS>{}, A, ws + L_DV, lane);
+  wave_sync();
+  lu_store(A, c, a21, dl, dt, opaque_lds(ws), opaque_lane(lane));
+}
+
+__device__ __forceinline__ void factor_2d(double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws, int lane) {
+  LuBlock A;
+  lu_load(A, c, a21, opaque_lds(ws), opaque_lane(lane));
+  lu_factor(A, c, a21, dl, dt, ws, lane);
+}
+
+// The LU of M0 by rows: the lead columns (right-looking, dense in LDS), the Schur update of the trailing block, then
+// the trailing block in registers. dl: 1 / U_ii of lead row lane; dt: of trailing row lane.
+__device__ __forceinline__ void factor_rows(double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
+                                            int lane) {
   factor_lead(c, a21, dl, ws, lane);
   factor_trailing(c, dt, ws, lane);
+}
+
+__device__ __forceinline__ void factor(double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws, int lane) {
+  if constexpr (LU_2D)
+    factor_2d(c, a21, dl, dt, ws, lane);
+  else
+    factor_rows(c, a21, dl, dt, ws, lane);
 }
 
 // y <- M0^-1 y for NV vectors (lead / trailing parts), with factor's factors, in three parts: the lead columns of L,
@@ -796,6 +1132,8 @@ __device__ __forceinline__ void solve_lead_backward(double (&yl)[NV], const doub
 template <int NV>
 __device__ __forceinline__ void solve(double (&yl)[NV], double (&yt)[NV], const double (&c)[NT], const LeadRow& a21,
                                       double dl, double dt, double* ws, int lane) {
+  ws = opaque_lds(ws);
+  lane = opaque_lane(lane);
   solve_lead_forward(yl, yt, a21, ws, lane);
   solve_trailing(yt, c, dt, lane);
   solve_lead_backward(yl, yt, dl, ws, lane);
