@@ -104,7 +104,7 @@ def lu_layout(tab: Tables) -> dict:
     """The two-dimensional LU's layout (kernels/common.hip, factor_2d): register slots of 16 rows (m) by 4 columns
     (t), the lead rows' and columns' (ml, tl) first; per pivot, the row slots that hold an entry below it in its column
     and the column slots that hold one right of it in its row, in the filled pattern; per row slot, the column slots
-    that hold any entry. The trailing rows' columns pass through the cell's LDS from its dv terms to its trash slots,
+    that hold any entry. The trailing rows' columns pass through the cell's LDS from its dv terms to its spare slots,
     chunk column slots of stride doubles a column at a time."""
     ns, k0, nt, fill, lay = tab.ns, tab.k0, tab.nt, tab.fill, tab.layout()
     ml, tl = -(-k0 // 16), -(-k0 // 4)
@@ -118,14 +118,14 @@ def lu_layout(tab: Tables) -> dict:
     rows = [bits(row[np.flatnonzero(fill[k + 1 :, k]) + k + 1]) for k in range(ns)]
     cols = [bits(col[np.flatnonzero(fill[k, k + 1 :]) + k + 1]) for k in range(ns)]
     live = [bits(col[np.flatnonzero(fill[row == r].any(0))]) for r in range(m)]
-    room = lay["TRASH"] + C.WAVE - lay["DV"]
+    room = lay["SPARE"] + C.WAVE - lay["DV"]
     stride = 16 * (m - ml)
     # 16 doubles more a column put neighbouring columns on other banks, where that costs no more chunks
     plain, wide = (min(t, room // (4 * q)) for q in (stride, stride + 16))
     if wide and -(-t // wide) == -(-t // plain):
         stride, plain = stride + 16, wide
     need = max(64 * m, 16 * m + 4 * tl + C.WAVE)  # the multipliers' exchange; the diagonal and its reciprocals
-    fits = plain > 0 and room >= need and 16 * ml * ns <= lay["TRASH"] + C.WAVE  # whole slots of lead rows are read
+    fits = plain > 0 and room >= need and 16 * ml * ns <= lay["SPARE"] + C.WAVE  # whole slots of lead rows are read
     return {"use": ns <= LU_MAX_SPECIES and fits, "m": m, "t": t, "ml": ml, "tl": tl,
             "rows": rows, "cols": cols, "live": live, "chunk": max(plain, 1), "stride": stride}  # fmt: skip
 
@@ -145,6 +145,7 @@ def header(tab: Tables, cpw: int, drift: float, batch: int = DEFAULT_BATCH, mixe
     ints = {
         "WAVE": C.WAVE, "NS": tab.ns, "NR": tab.nr, "NRT": tab.nrt, "NJ": tab.nj, "K0": tab.k0, "NT": tab.nt,
         "NEL": tab.nel, "RCW": C.RATE_ROW, "RROUNDS": -(-tab.nr // C.WAVE), "NDV": tab.ndv, "NPART": tab.npart,
+        "PIECE_MAX": max(1, int((tab.row_pieces >> 16).max(initial=0))),
         "CPW": cpw, "STREAM_BATCH": batch, "REC_WAVES": REC_WAVES, "CHUNK": CHUNK,
         "NCH": nch, "NLCH": tab.nlch,
         "SV_ROUNDS": tab.sv_words.shape[0], "DIAG_ROUNDS": tab.diag_words.shape[0],
@@ -231,20 +232,40 @@ def lds_bytes(tab: Tables, cpw: int, mixed: bool = False, rates_global: bool = F
     return 8 * size * cpw + words, 8 * (size + tab.ns * tab.ns + 2 * tab.ns) + 4 * tab.ns + 4
 
 
+def every_destination(words: np.ndarray, end: int, dest: int, spare: np.ndarray) -> np.ndarray:
+    """A stream's words [rounds, lanes] with the destination of the entry they belong to in every word (the tables hold
+    it in the entry's last word, which keeps its mark). A lane's padding words take its last entry's, or spare[lane]."""
+    low = np.uint32((1 << dest) - 1)
+    field = np.uint32(0x7FFFFFFF) & ~low  # the destination's bits: from dest to the sign bit
+    out = words.copy()
+    for lane in range(words.shape[1]):
+        place = np.uint32(int(spare[lane]) << dest)
+        ends = np.flatnonzero(words[:, lane] >> np.uint32(end) & 1)
+        if len(ends):
+            place = words[ends[-1], lane] & field
+        for r in range(words.shape[0] - 1, -1, -1):
+            if words[r, lane] >> np.uint32(end) & 1:
+                place = words[r, lane] & field
+            out[r, lane] = (words[r, lane] & ~field) | place
+    return out
+
+
 def host_tables(tab: Tables) -> dict[str, np.ndarray]:
     """The tables the kernels read through their Net struct, as contiguous host arrays (species in elimination
     order where the kernels index them so)."""
+    spare = tab.layout()["DIAG"] + np.arange(C.WAVE) % tab.nt
     t = {
         "perm": tab.perm.astype(np.int32),
         "rc": tab.rc.astype(np.float64),
         "rf": tab.rf.astype(np.int32),
         "nasa": tab.nasa[:, tab.perm, :].astype(np.float64),
         "rxe": tab.rxe.view(np.int64),
-        "svw": tab.sv_words.ravel().view(np.int32),
+        "svw": every_destination(tab.sv_words, SV_END, SV_PIECE, np.arange(C.WAVE) % tab.npart).ravel().view(np.int32),
         "rowp": tab.row_pieces.view(np.int32),
-        "diagw": tab.diag_words.ravel().view(np.int32),
-        "leadw": tab.lead_words.ravel().view(np.int32),
-        "chw": np.concatenate([w.ravel() for w in tab.chunk_words]).view(np.int32),
+        "diagw": every_destination(tab.diag_words, T_END, T_DEST, spare).ravel().view(np.int32),
+        "leadw": every_destination(tab.lead_words, T_END, T_DEST, spare).ravel().view(np.int32),
+        "chw": np.concatenate([every_destination(w, T_END, T_DEST, spare).ravel() for w in tab.chunk_words]).view(
+            np.int32),
         "atoms": tab.atoms.astype(np.float64),
         "rord": tab.rord.astype(np.int32),
     }

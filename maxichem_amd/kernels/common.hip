@@ -155,13 +155,16 @@ __device__ __forceinline__ double coefficient(u32 w, int neg, int dbl) {
 }
 
 // A stream word's term: d times the word's coefficient, exactly as fma(coefficient, d, .) takes it: x2 is an exponent
-// step, and the sign (the word's bit 31) is XORed into the double's sign bit. Four instructions, where the
-// coefficient's compares and selects take eight and wait states for their condition masks.
+// step, and the sign (the word's bit 31) is XORed into the double's sign bit, or put there where d is not SIGNED (then
+// one instruction). No compares and selects, and no wait states for condition masks.
 static_assert(T_NEG == 31 && SV_NEG == 31, "the streams' sign bit is the word's sign bit");
-template <int DBL>
+template <int DBL, bool SIGNED = true>
 __device__ __forceinline__ double term(u32 w, double d) {
   d = __builtin_amdgcn_ldexp(d, (int)((w >> DBL) & 1u));
-  return __longlong_as_double(__double_as_longlong(d) ^ ((long long)(w & 0x80000000u) << 32));
+  const long long b = __double_as_longlong(d);
+  const u32 hi = (u32)((u64)b >> 32);
+  const u32 h = SIGNED ? hi ^ (w & 0x80000000u) : (hi & 0x7fffffffu) | (w & 0x80000000u);
+  return __longlong_as_double((long long)((u64)h << 32 | (u32)b));
 }
 
 // A table pointer in the global address space. Loads through it are global loads, counted by the vector-memory
@@ -310,17 +313,22 @@ __device__ __forceinline__ void cell_rates(double* ws, double* rk, double T, dou
 
 // ---- right-hand side and Jacobian ----
 
-// A term stream (the Jacobian's and S v's): each lane sums whole entries from src terms and writes each at its
-// destination in dst. The words of STREAM_BATCH rounds are loaded together, ahead of their terms, so that their
-// latency is paid once per batch: whole batches in a loop, then the last rounds as a batch of their own (the rounds
-// are known when the kernel is built, so no padding terms are taken). Every word stores the running sum, at its
-// entry's destination when it ends one and else in the lane's trash slot, and the sum restarts where an entry ended:
-// no branch and no exec-mask change per word. (Loading each batch, or a stream's first batch, one step ahead was
-// measured slower: it holds 36 more registers.)
-template <unsigned IDX_MASK, int DBL, int END, int DEST, unsigned DEST_MASK, typename WP>
+// d added to the double at p in LDS, in the order of the wave's LDS accesses (ds_add_f64, rounded as a vector add).
+__device__ __forceinline__ void lds_add(double* p, double d) {
+  __hip_atomic_fetch_add((__attribute__((address_space(3))) double*)p, d, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// A term stream (the Jacobian's and S v's): each lane adds the terms of whole entries, in their order, to the entries'
+// places in dst, which hold 0 before (padding words add 0 to a place of their lane's). The adds are LDS atomics: an
+// entry's terms come from one lane, so they are taken in order, and a word costs no running sum, no select and no
+// wait: 9 instructions, where a running sum with its selects took 19 (NCHO, cycles of one wavefront per try: the
+// Jacobian 23.0k -> 17.4k, the three right-hand sides 21.4k -> 17.9k). The words of STREAM_BATCH rounds are loaded together, ahead of their terms, so that their latency is paid once
+// per batch: whole batches in a loop, then the last rounds as a batch of their own (the rounds are known when the kernel
+// is built). SIGNED: the terms may be negative; else the word's sign bit is put in place of theirs.
+template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, bool SIGNED, typename WP>
 __device__ __forceinline__ void stream_sum(WP __restrict__ words, int rounds, const double* src, double* dst,
-                                           double* trash, int lane) {
-  double acc = 0.0;
+                                           int lane) {
   auto batch = [&](int q0, int n) {  // rounds q0 .. q0 + n - 1, n <= STREAM_BATCH
     u32 w[STREAM_BATCH];
     double d[STREAM_BATCH];
@@ -333,10 +341,7 @@ __device__ __forceinline__ void stream_sum(WP __restrict__ words, int rounds, co
 #pragma unroll
     for (int i = 0; i < STREAM_BATCH; i++) {
       if (i >= n) break;
-      acc += term<DBL>(w[i], d[i]);
-      const bool end = (w[i] >> END) & 1u;
-      *(end ? dst + ((w[i] >> DEST) & DEST_MASK) : trash) = acc;
-      acc = end ? 0.0 : acc;
+      lds_add(dst + ((w[i] >> DEST) & DEST_MASK), term<DBL, SIGNED>(w[i], d[i]));
     }
   };
   const int full = rounds / STREAM_BATCH * STREAM_BATCH;
@@ -348,7 +353,7 @@ __device__ __forceinline__ void stream_sum(WP __restrict__ words, int rounds, co
 // One Jacobian stream into the cell's LDS: entries of -Jn at their offsets.
 template <typename WP>
 __device__ __forceinline__ void jac_stream(WP __restrict__ words, int rounds, const double* DV, double* ws, int lane) {
-  stream_sum<T_IDX_MASK, T_DBL, T_END, T_DEST, T_DEST_MASK>(words, rounds, DV, ws, ws + L_TRASH + lane, lane);
+  stream_sum<T_IDX_MASK, T_DBL, T_DEST, T_DEST_MASK, false>(words, rounds, DV, ws, lane);  // dv terms are not negative
 }
 
 // The stream words in the workgroup's LDS (WORDS_LDS: the call kernel copies them there at its start, after its
@@ -421,29 +426,35 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
       }
     }
   }
+  double* part = ws + L_PART;
+#pragma unroll
+  for (int i = 0; i < NPART; i += WAVE)
+    if (i + lane < NPART) part[i + lane] = 0.0;
   if (lane == 0) V[NR] = 0.0;  // the S v stream's padding term
   wave_sync();
-  double* part = ws + L_PART;
   if constexpr (LW)
-    stream_sum<SV_R_MASK, SV_DBL, SV_END, SV_PIECE, SV_PIECE_MASK>(lds_words(ws) + W_SV, SV_ROUNDS, V, part,
-                                                                  ws + L_TRASH + lane, lane);
+    stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true>(lds_words(ws) + W_SV, SV_ROUNDS, V, part, lane);
   else
-    stream_sum<SV_R_MASK, SV_DBL, SV_END, SV_PIECE, SV_PIECE_MASK>(svw, SV_ROUNDS, V, part, ws + L_TRASH + lane,
-                                                                  lane);
+    stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true>(svw, SV_ROUNDS, V, part, lane);
   wave_sync();
-  if (lane < K0) {
-    double s = 0.0;
-    for (int e = 0; e < (int)(rpl >> 16); e++) s += part[(rpl & 0xffffu) + e];
-    Fl = s * ixf;
-    u0l = s / nd;
+  // each row's pieces in order; the reads go out together (a row of fewer pieces than the most reads within part)
+  auto row = [&](u32 rp) {
+    const int first = (int)(rp & 0xffffu), count = (int)(rp >> 16);
+    double v[PIECE_MAX], s = 0.0;
+#pragma unroll
+    for (int e = 0; e < PIECE_MAX; e++) v[e] = part[e < count ? first + e : 0];
+#pragma unroll
+    for (int e = 0; e < PIECE_MAX; e++) s = e < count ? s + v[e] : s;
+    return s;
+  };
+  if (K0 > 0) {
+    const double s = row(rpl);
+    Fl = lane < K0 ? s * ixf : Fl;
+    u0l = lane < K0 ? s / nd : u0l;
   }
-  if (lane < NT) {
-    const u32 rp = rpt;
-    double s = 0.0;
-    for (int e = 0; e < (int)(rp >> 16); e++) s += part[(rp & 0xffffu) + e];
-    Ft = s * ixf;
-    u0t = s / nd;
-  }
+  const double s = row(rpt);
+  Ft = lane < NT ? s * ixf : Ft;
+  u0t = lane < NT ? s / nd : u0t;
   wave_sync();
   return ntot;
 }
