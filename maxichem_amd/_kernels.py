@@ -32,7 +32,10 @@ from ._tables import (
 KERNEL_DIR = Path(__file__).resolve().parent / "kernels"
 KERNEL_FILES = ("common.hip", "guard.hip", "call.hip", "recover.hip")
 ARCH = "gfx950"
-# hiprtc options: gfx950 code; packed FP32 instructions are kept out of all code (a known hazard on these parts)
+# hiprtc options: gfx950 code; packed FP32 instructions are kept out of all code (a known hazard on these parts);
+# constants and addresses stay in the loops that use them (hoisted out of the loops over cells and tries, they are held
+# in registers across a whole try or spilled: the call kernel on NCHO takes 276 registers instead of 332, and at two
+# wavefronts per SIMD spills 76 bytes per lane instead of 300)
 OPTIONS = (
     f"--offload-arch={ARCH}",
     "-O3",
@@ -42,6 +45,8 @@ OPTIONS = (
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
+    "-mllvm",
+    "-disable-machine-licm",
 )
 REC_WAVES = 4  # wavefronts of a recovery workgroup: the first steps the cell, all of them share its dense LU
 KERNEL_NAMES = ("mxc_call", "mxc_recover")

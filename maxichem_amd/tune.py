@@ -27,11 +27,16 @@ CU_WAVES = 4  # call wavefronts per compute unit at one per SIMD
 
 
 def default_variant(tab, mixed: bool = False) -> tuple[int, int, int, int]:
-    """The variant without a stored choice, with the same bits as every other: four cells per workgroup when the
-    stream words then fit in the workgroup's LDS at as many cells per compute unit (on MI355X 2.6 % faster on NCHO:
-    the words come with the LDS's latency instead of the caches'); else two when that keeps as many cells per
-    compute unit as one (about 2 % faster: single-wavefront workgroups leave the SIMDs less evenly loaded); else
-    one."""
+    """The variant without a stored choice, with the same bits as every other. Two wavefronts per SIMD where a compute
+    unit's LDS holds eight cells (with the rates in LDS, else in global scratch): each waits for its LDS reads and
+    chains of broadcasts while the other issues, which outweighs the few registers it spills (NCHO, kernel ms: 8,192
+    cold cells 45.2 -> 32.4, 65,536 settled cells 12.5 -> 12.0, 256 cold cells 20.4 -> 18.7). Else, and in the mixed
+    form: four cells per workgroup when the stream words then fit in the workgroup's LDS at as many cells per compute
+    unit; else two when that keeps as many cells per compute unit as one; else one."""
+    if not mixed and _kernels.lu_layout(tab)["use"]:
+        for rates_global in (0, 1):
+            if CU_LDS // _kernels.lds_bytes(tab, 1, False, bool(rates_global), 2)[0] >= 2 * CU_WAVES:
+                return (1, _kernels.DEFAULT_BATCH, 2, rates_global)
 
     def cells(cpw: int) -> int:
         return min(CU_WAVES, CU_LDS // _kernels.lds_bytes(tab, cpw, mixed)[0] * cpw)
