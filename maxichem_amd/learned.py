@@ -56,6 +56,30 @@ class Layer:
     gb: torch.Tensor
 
 
+FUSED_WIDTH, FUSED_LAYERS = 256, 8  # the one-launch kernels' limits (kernels/mlp.hip)
+_P8, _I8 = ctypes.c_void_p * FUSED_LAYERS, ctypes.c_int * FUSED_LAYERS
+
+
+class _Layers(ctypes.Structure):
+    _fields_ = [("W", _P8), ("bias", _P8), ("z", _P8), ("act", _P8), ("K", _I8), ("N", _I8), ("layers", ctypes.c_int),
+                ("M", ctypes.c_int)]  # fmt: skip
+
+
+class _Transposes(ctypes.Structure):
+    _fields_ = [("W", _P8), ("T", _P8), ("K", _I8), ("N", _I8), ("layers", ctypes.c_int)]
+
+
+class _Gradients(ctypes.Structure):
+    _fields_ = [("dz", _P8), ("x", _P8), ("gw", _P8), ("gb", _P8), ("K", _I8), ("N", _I8), ("layers", ctypes.c_int),
+                ("M", ctypes.c_int), ("splits", ctypes.c_int), ("rows", ctypes.c_int), ("partial", ctypes.c_void_p),
+                ("total", ctypes.c_long)]  # fmt: skip
+
+
+def _pointers(tensors):
+    """Device pointers of up to FUSED_LAYERS tensors (None: null) as a kernel argument's array."""
+    return _P8(*[None if a is None else a.data_ptr() for a in tensors])
+
+
 class MLP:
     """An MLP of n_in -> width x depth (GELU) -> n_out on one device, padded to the kernels' tiles."""
 
@@ -77,7 +101,10 @@ class MLP:
         self._mod = module(self.dev.index if self.dev.index is not None else torch.cuda.current_device())
         self._fn = {name: self._mod.function(name) for name in (
             "mlp_gemm_f32", "mlp_gemm_bias_gelu", "mlp_gemm_bias", "mlp_loss", "mlp_gelu_backward",
-            "mlp_column_sum", "mlp_column_total", "mlp_adam", "mlp_to_bf16")}  # fmt: skip
+            "mlp_column_sum", "mlp_column_total", "mlp_adam", "mlp_to_bf16", "mlp_forward_32", "mlp_forward_64",
+            "mlp_backward_32", "mlp_transposes", "mlp_gradients", "mlp_gradient_sums")}  # fmt: skip
+        # the whole network in one launch where its layers fit a workgroup's LDS tile; else a launch per layer
+        self.fused = max(self.dims) <= FUSED_WIDTH and depth + 1 <= FUSED_LAYERS
         self.loss = torch.zeros(1, dtype=torch.float32, device=self.dev)
         self._sync_bf16()
 
@@ -110,6 +137,8 @@ class MLP:
     def forward(self, X: torch.Tensor, keep: bool = False) -> torch.Tensor:
         """Y [M, n_out_pad] FP32 of the BF16 inputs X [M, n_in_pad] (int16 storage); M a multiple of 64."""
         M = X.shape[0]
+        if self.fused:
+            return self._forward_fused(X, keep)
         p = _hip.ptr
         a = X
         acts, pre = [X], []
@@ -130,8 +159,66 @@ class MLP:
             self._acts, self._pre = acts, pre
         return y
 
+    def _forward_fused(self, X: torch.Tensor, keep: bool) -> torch.Tensor:
+        """forward in one launch: 64 rows a workgroup, or 32 where 64 would leave compute units idle (fewer than two
+        workgroups each). On MI355X, 65,536 rows of the 120 -> 4 x 256 -> 71 network: 119 us, from 216 a layer at a
+        time, of which the erf of GELU takes most."""
+        M = X.shape[0]
+        assert M % TILE == 0 and X.shape[1] == self.dims[0], (X.shape, self.dims)
+        d, n = self.dims, self.depth + 1
+
+        def empty(dtype, count, wanted=True):
+            return [torch.empty(M, d[l + 1], dtype=dtype, device=self.dev) if wanted else None for l in range(count)]
+
+        y = torch.empty(M, d[-1], dtype=torch.float32, device=self.dev)
+        pre, acts = empty(torch.float32, self.depth, keep), empty(torch.int16, self.depth, keep)
+        args = _Layers(_pointers([ly.wb for ly in self.layers]), _pointers([ly.b for ly in self.layers]),
+                       _pointers([*pre, y]), _pointers([*acts, None]), _I8(*d[:-1]), _I8(*d[1:]), n, M)  # fmt: skip
+        rows = 64 if M >= 64 * 512 else 32
+        if M:
+            _hip.launch(self._fn[f"mlp_forward_{rows}"], -(-M // rows), 512, 0, self._stream(), [_hip.ptr(X), args])
+        if keep:
+            self._acts, self._pre = [X, *acts], pre
+        return y
+
+    def _backward_fused(self, dY: torch.Tensor) -> None:
+        """backward in four launches: the weights' transposes, every layer's dz, the gradients' parts over splits of the
+        samples, and their sums. On MI355X, 8,192 rows of the 120 -> 4 x 256 -> 71 network: 74 us, from about 3 ms with
+        one workgroup per 64 x 64 tile of a gradient."""
+        M, d, n = dY.shape[0], self.dims, self.depth + 1
+        assert M % TILE == 0 and dY.shape[1] == d[-1], (dY.shape, d)
+        f32, stream = {"dtype": torch.float32, "device": self.dev}, self._stream()
+        if not M:
+            for ly in self.layers:
+                ly.gw.zero_()
+                ly.gb.zero_()
+            return
+        K, N = _I8(*d[:-1]), _I8(*d[1:])
+        wt = [torch.empty(d[l], d[l + 1], dtype=torch.int16, device=self.dev) if l else None for l in range(n)]
+        tr = _Transposes(_pointers([ly.wb for ly in self.layers[1:]]), _pointers(wt[1:]), _I8(*d[1:-1]), _I8(*d[2:]),
+                         n - 1)  # fmt: skip
+        tiles = sum((d[l] // TILE) * (d[l + 1] // TILE) for l in range(1, n))
+        dz = [torch.empty(M, d[l + 1], dtype=torch.int16, device=self.dev) for l in range(self.depth)] + [dY]
+        if self.depth:
+            _hip.launch(self._fn["mlp_transposes"], tiles, 256, 0, stream, [tr])
+            back = _Layers(_pointers(wt), _P8(), _pointers(self._pre), _pointers(dz), K, N, n, M)
+            _hip.launch(self._fn["mlp_backward_32"], -(-M // 32), 512, 0, stream, [_hip.ptr(dY), back])
+        # about 512 samples a split, at most 16 splits (each split's parts are written and read once more)
+        splits = max(1, min(16, M // 512))
+        rows = pad(-(-M // splits))
+        total = sum(d[l] * d[l + 1] + d[l + 1] for l in range(n))
+        partial = torch.empty(splits, total, **f32)
+        g = _Gradients(_pointers(dz), _pointers(self._acts), _pointers([ly.gw for ly in self.layers]),
+                       _pointers([ly.gb for ly in self.layers]), K, N, n, M, splits, rows, partial.data_ptr(), total)  # fmt: skip
+        tiles = sum(-(-d[l] // 128) * -(-d[l + 1] // 128) for l in range(n))
+        _hip.launch(self._fn["mlp_gradients"], tiles * splits, 256, 0, stream, [g])
+        _hip.launch(self._fn["mlp_gradient_sums"], -(-total // 1024), 256, 0, stream, [g])
+
     def backward(self, dY: torch.Tensor) -> None:
         """Gradients of every layer (gw, gb) from dY [M, n_out_pad] (BF16) after forward(keep=True)."""
+        if self.fused:
+            self._backward_fused(dY)
+            return
         M = dY.shape[0]
         p = _hip.ptr
         dz = dY
@@ -162,8 +249,9 @@ class MLP:
         M, ldy = Y.shape
         dY = torch.empty(M, ldy, dtype=torch.int16, device=self.dev)
         p = _hip.ptr
-        self._elementwise("mlp_loss", M * ldy, [p(Y), p(T), p(w), ctypes.c_int(rows), ctypes.c_int(self.n_out),
-                                                ctypes.c_long(ldy), ctypes.c_long(M * ldy), p(dY), p(self.loss)])  # fmt: skip
+        _hip.launch(self._fn["mlp_loss"], max(1, min(512, -(-M * ldy // 256))), 256, 0, self._stream(),
+                    [p(Y), p(T), p(w), ctypes.c_int(rows), ctypes.c_int(self.n_out), ctypes.c_long(ldy),
+                     ctypes.c_long(M * ldy), p(dY), p(self.loss)])  # fmt: skip
         return dY
 
     def adam(self, lr: float, beta1: float = 0.9, beta2: float = 0.999, eps: float = 1e-8, decay: float = 0.0) -> None:
