@@ -17,7 +17,7 @@ template <int NV>
 __device__ __forceinline__ bool solve_m0(double (&yl)[NV], double (&yt)[NV], const double (&c)[NT],
                                          const LeadRow& a21, double dl, double dtr, double, double, double,
                                          NetP, double* ws, int lane) {
-  solve<NV>(yl, yt, c, a21, dl, dtr, ws, lane);
+  solve<NV, BLOCK_SOLVES>(yl, yt, c, a21, dl, dtr, ws, lane);
   return true;
 }
 
@@ -57,7 +57,7 @@ __device__ __forceinline__ bool stages(T (&c)[NT], LeadRow& a21, double Nl, doub
   if constexpr (LU_2D && sizeof(T) == sizeof(double)) {
     LuBlock A;
     lu_assemble<WORDS_LDS != 0>(A, igh, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
-    lu_factor(A, c, a21, dl, dtr, ws, lane);
+    lu_factor<BLOCK_SOLVES>(A, c, a21, dl, dtr, ws, lane);
   } else {
     jacobian<WORDS_LDS != 0>(c, a21, Nl, Nt, u0l, u0t, ntot, ul, ut, net, ws, lane);
     add_diagonal(c, igh, ws, lane);

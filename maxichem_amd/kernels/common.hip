@@ -874,6 +874,8 @@ __device__ __forceinline__ void lu_load(LuBlock& A, const double (&c)[NT], const
 
 // The factors out of A: 1 / U_ii of lead row lane (dl) and of trailing row lane (dt); each column times its 1 / U_jj
 // below the diagonal (L) and, in the trailing rows, above it (U' = U diag(1 / U_jj)); and the rows back to their lanes.
+// ZERO: the trailing diagonal as 0 (for solve_blocks), else U_ii.
+template <bool ZERO>
 __device__ __forceinline__ void lu_store(LuBlock& A, double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
                                          int lane) {
   const LuPlace p(ws, lane);
@@ -910,6 +912,7 @@ __device__ __forceinline__ void lu_store(LuBlock& A, double (&c)[NT], LeadRow& a
       const bool diag = m < LU_ML ? t < LU_TL && t / 4 == m : t >= LU_TL && (t - LU_TL) / 4 == m - LU_ML;
       const int j = 4 * (m < LU_ML ? t & 3 : (t - LU_TL) & 3) + g;  // the column's row in a diagonal slot
       A[m][t] *= !diag || s > j || (m >= LU_ML && s != j) ? d : 1.0;
+      if (ZERO && diag && m >= LU_ML) A[m][t] = s == j ? 0.0 : A[m][t];
     }
   }
   wave_sync();
@@ -989,19 +992,20 @@ __device__ __forceinline__ void lu_assemble(LuBlock& A, double igh, double Nl, d
 }
 
 // The LU of A into the rows by lane, and the reciprocals of its diagonal.
+template <bool ZERO>
 __device__ __forceinline__ void lu_factor(LuBlock& A, double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
                                           int lane) {
   lane = opaque_lane(lane);
   ws = opaque_lds(ws);
   lu_steps(Steps<NS>{}, A, ws + L_DV, lane);
   wave_sync();
-  lu_store(A, c, a21, dl, dt, opaque_lds(ws), opaque_lane(lane));
+  lu_store<ZERO>(A, c, a21, dl, dt, opaque_lds(ws), opaque_lane(lane));
 }
 
 __device__ __forceinline__ void factor_2d(double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws, int lane) {
   LuBlock A;
   lu_load(A, c, a21, opaque_lds(ws), opaque_lane(lane));
-  lu_factor(A, c, a21, dl, dt, ws, lane);
+  lu_factor<false>(A, c, a21, dl, dt, ws, lane);
 }
 
 // The LU of M0 by rows: the lead columns (right-looking, dense in LDS), the Schur update of the trailing block, then
@@ -1021,17 +1025,28 @@ __device__ __forceinline__ void factor(double (&c)[NT], LeadRow& a21, double& dl
 
 // y <- M0^-1 y for NV vectors (lead / trailing parts), with factor's factors, in three parts: the lead columns of L,
 // the trailing block, the lead rows of U.
+constexpr int LEAD_BATCH = 14;  // lead columns read ahead of their steps
+
 template <int NV>
 __device__ __forceinline__ void solve_lead_forward(double (&yl)[NV], double (&yt)[NV], const LeadRow& a21,
                                                    const double* ws, int lane) {
+  const double* row = ws + (lane < K0 ? lane : 0) * NS;  // in bounds for every lane, so that no read waits on a branch
 #pragma unroll
-  for (int k = 0; k < K0; k++) {  // unit L, lead columns (the trailing rows' entries in a21)
-    const double lk = (lane > k && lane < K0) ? ws[lane * NS + k] : 0.0;
+  for (int k0 = 0; k0 < K0; k0 += LEAD_BATCH) {  // unit L, lead columns (the trailing rows' entries in a21)
+    double l[LEAD_BATCH];
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      const double yk = readlane(yl[v], k);
-      yl[v] = fma(-lk, yk, yl[v]);
-      yt[v] = fma(-a21[k], yk, yt[v]);
+    for (int i = 0; i < LEAD_BATCH; i++) l[i] = k0 + i < K0 ? row[k0 + i] : 0.0;
+#pragma unroll
+    for (int i = 0; i < LEAD_BATCH; i++) {
+      const int k = k0 + i;
+      if (k >= K0) break;
+      const double lk = (lane > k && lane < K0) ? l[i] : 0.0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        const double yk = readlane(yl[v], k);
+        yl[v] = fma(-lk, yk, yl[v]);
+        yt[v] = fma(-a21[k], yk, yt[v]);
+      }
     }
   }
 }
@@ -1079,6 +1094,28 @@ __device__ __forceinline__ void solve_trailing(double (&yt)[NV], const double (&
   for (int v = 0; v < NV; v++) yt[v] *= dt;
 }
 
+// U of the lead rows, lead columns.
+template <int NV>
+__device__ __forceinline__ void solve_lead_upper(double (&yl)[NV], double dl, const double* ws, int lane) {
+  const double* row = ws + (lane < K0 ? lane : 0) * NS;
+#pragma unroll
+  for (int k1 = K0; k1 > 0; k1 -= LEAD_BATCH) {
+    double u[LEAD_BATCH];
+#pragma unroll
+    for (int i = 0; i < LEAD_BATCH; i++) u[i] = k1 - 1 - i >= 0 ? row[k1 - 1 - i] : 0.0;
+#pragma unroll
+    for (int i = 0; i < LEAD_BATCH; i++) {
+      const int k = k1 - 1 - i;
+      if (k < 0) break;
+      const double uk = lane < k ? u[i] : 0.0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) yl[v] = fma(-uk, readlane(yl[v] * dl, k), yl[v]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; v++) yl[v] *= dl;
+}
+
 template <int NV>
 __device__ __forceinline__ void solve_lead_backward(double (&yl)[NV], const double (&yt)[NV], double dl, double* ws,
                                                     int lane) {
@@ -1087,7 +1124,7 @@ __device__ __forceinline__ void solve_lead_backward(double (&yl)[NV], const doub
     double sum[K0 > 0 ? K0 * NV : 1];
 #pragma unroll
     for (int i = 0; i < K0; i++) {
-      const double a = lane < NT ? ws[i * NS + K0 + lane] : 0.0;
+      const double a = NT == WAVE || lane < NT ? ws[i * NS + K0 + lane] : 0.0;
 #pragma unroll
       for (int v = 0; v < NV; v++) sum[i * NV + v] = a * yt[v];
     }
@@ -1097,14 +1134,7 @@ __device__ __forceinline__ void solve_lead_backward(double (&yl)[NV], const doub
 #pragma unroll
       for (int v = 0; v < NV; v++) yl[v] = lane == i ? yl[v] - sum[i * NV + v] : yl[v];
     }
-#pragma unroll
-    for (int k = K0 - 1; k >= 0; k--) {  // U, lead columns
-      const double uk = lane < k ? ws[lane * NS + k] : 0.0;
-#pragma unroll
-      for (int v = 0; v < NV; v++) yl[v] = fma(-uk, readlane(yl[v] * dl, k), yl[v]);
-    }
-#pragma unroll
-    for (int v = 0; v < NV; v++) yl[v] *= dl;
+    solve_lead_upper(yl, dl, ws, lane);
   } else if (K0 > 0) {
     // U of the lead rows, trailing columns: the trailing solution through LDS (the union region is free between
     // the right-hand sides), a batch of columns at a time
@@ -1129,24 +1159,156 @@ __device__ __forceinline__ void solve_lead_backward(double (&yl)[NV], const doub
       }
     }
     wave_sync();
-#pragma unroll 1
-    for (int k = K0 - 1; k >= 0; k--) {  // U, lead columns
-      const double uk = lane < k ? ws[lane * NS + k] : 0.0;
+    solve_lead_upper(yl, dl, ws, lane);
+  }
+}
+
+// The trailing solves by blocks of 16 rows, one row of lanes each, for a full trailing block (NT == WAVE) whose c has 0
+// on the diagonal. Within a block, lane k's value reaches its row of lanes by DPP inside the fma, and the exec mask
+// keeps the lanes already final (their c entries belong to the other triangle); a finished block reaches the other
+// rows of lanes through LDS, and its 16 updates there take it by DPP too. An entry takes its updates in the order of
+// solve_trailing, so the bits are the same. A step costs 3 issue slots for one vector and 3 for two (an exec shift, an
+// fma each, a wait), an update of the other rows one, where a step by v_readlane and v_writelane takes 7 and 11.
+// Cycles of one wavefront (NCHO, the lead rows' part included): one vector 5.7k -> 4.1k, two 9.7k -> 5.9k; on
+// SNCHO, whose 27 lead columns are now read ahead of their steps, 13.6k -> 8.6k and 20.9k -> 13.5k.
+// (DPP reads a register two wait states after a vector instruction wrote it: the other vector's fma and the exec shift,
+// or s_nop; the blocks' first and last instructions keep the same distance from the compiler's.)
+#define MXC_FWD "s_lshl_b64 exec, exec, 1\n\t"
+#define MXC_BWD "s_lshr_b64 exec, exec, 1\n\t"
+#define MXC_DPP(Y, X, K, ROWS) "v_fmac_f64_dpp %[" Y "], %[" X "], -%[c" #K "] row_newbcast:" #K " row_mask:" ROWS " bank_mask:0xf\n\t"
+#define MXC_ST1(MOVE, K, ROWS) MOVE "s_nop 0\n\t" MXC_DPP("y", "y", K, ROWS)
+#define MXC_ST2(MOVE, K, ROWS) MOVE MXC_DPP("y", "y", K, ROWS) MXC_DPP("z", "z", K, ROWS)
+#define MXC_UP1(MOVE, K, ROWS) MXC_DPP("y", "p", K, ROWS)
+#define MXC_UP2(MOVE, K, ROWS) MXC_DPP("y", "p", K, ROWS) MXC_DPP("z", "q", K, ROWS)
+#define MXC_ASC(S, M, R)                                                                                        \
+  S("", 0, R) S(M, 1, R) S(M, 2, R) S(M, 3, R) S(M, 4, R) S(M, 5, R) S(M, 6, R) S(M, 7, R) S(M, 8, R) S(M, 9, R) \
+  S(M, 10, R) S(M, 11, R) S(M, 12, R) S(M, 13, R) S(M, 14, R)
+#define MXC_DESC(S, M, R)                                                                                         \
+  S("", 15, R) S(M, 14, R) S(M, 13, R) S(M, 12, R) S(M, 11, R) S(M, 10, R) S(M, 9, R) S(M, 8, R) S(M, 7, R) S(M, 6, R) \
+  S(M, 5, R) S(M, 4, R) S(M, 3, R) S(M, 2, R) S(M, 1, R)
+#define MXC_COLUMNS                                                                                               \
+  [c0] "v"(c[0]), [c1] "v"(c[1]), [c2] "v"(c[2]), [c3] "v"(c[3]), [c4] "v"(c[4]), [c5] "v"(c[5]), [c6] "v"(c[6]),  \
+      [c7] "v"(c[7]), [c8] "v"(c[8]), [c9] "v"(c[9]), [c10] "v"(c[10]), [c11] "v"(c[11]), [c12] "v"(c[12]),        \
+      [c13] "v"(c[13]), [c14] "v"(c[14]), [c15] "v"(c[15])
+// a block's own steps: exec shifted to its lanes (SHIFT), then one place a step
+#define MXC_OWN(ST, ORDER, MOVE, SHIFT, ROWS, ...)                                                                 \
+  asm volatile("s_mov_b64 %[e], exec\n\t" SHIFT "\n\ts_nop 1\n\t" ORDER(ST, MOVE, ROWS) "s_mov_b64 exec, %[e]\n\ts_nop 1" \
+               : __VA_ARGS__, [e] "=&s"(e)                                                                         \
+               : MXC_COLUMNS                                                                                      \
+               : "scc")
+#define MXC_OTHERS(UP, ORDER, LAST, ROWS, OUT, ...) \
+  asm volatile("s_nop 1\n\t" ORDER(UP, "", ROWS) UP("", LAST, ROWS) "s_nop 1" : OUT : __VA_ARGS__, MXC_COLUMNS)
+
+template <int B, bool UP>
+__device__ __forceinline__ void block_own(double (&yt)[1], const double* c) {
+  u64 e;
+#define MXC_OWN1(ORDER, MOVE, SHIFT, ROWS) MXC_OWN(MXC_ST1, ORDER, MOVE, SHIFT, ROWS, [y] "+&v"(yt[0]))
+  if constexpr (!UP) {
+    if constexpr (B == 0) MXC_OWN1(MXC_ASC, MXC_FWD, "s_nop 0", "0x1");
+    if constexpr (B == 1) MXC_OWN1(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 16", "0x2");
+    if constexpr (B == 2) MXC_OWN1(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 32", "0x4");
+    if constexpr (B == 3) MXC_OWN1(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 48", "0x8");
+  } else {
+    if constexpr (B == 0) MXC_OWN1(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 48", "0x1");
+    if constexpr (B == 1) MXC_OWN1(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 32", "0x2");
+    if constexpr (B == 2) MXC_OWN1(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 16", "0x4");
+    if constexpr (B == 3) MXC_OWN1(MXC_DESC, MXC_BWD, "s_nop 0", "0x8");
+  }
+}
+template <int B, bool UP>
+__device__ __forceinline__ void block_own(double (&yt)[2], const double* c) {
+  u64 e;
+#define MXC_OWN2(ORDER, MOVE, SHIFT, ROWS) MXC_OWN(MXC_ST2, ORDER, MOVE, SHIFT, ROWS, [y] "+&v"(yt[0]), [z] "+&v"(yt[1]))
+  if constexpr (!UP) {
+    if constexpr (B == 0) MXC_OWN2(MXC_ASC, MXC_FWD, "s_nop 0", "0x1");
+    if constexpr (B == 1) MXC_OWN2(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 16", "0x2");
+    if constexpr (B == 2) MXC_OWN2(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 32", "0x4");
+    if constexpr (B == 3) MXC_OWN2(MXC_ASC, MXC_FWD, "s_lshl_b64 exec, exec, 48", "0x8");
+  } else {
+    if constexpr (B == 0) MXC_OWN2(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 48", "0x1");
+    if constexpr (B == 1) MXC_OWN2(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 32", "0x2");
+    if constexpr (B == 2) MXC_OWN2(MXC_DESC, MXC_BWD, "s_lshr_b64 exec, exec, 16", "0x4");
+    if constexpr (B == 3) MXC_OWN2(MXC_DESC, MXC_BWD, "s_nop 0", "0x8");
+  }
+}
+
+template <int B, bool UP>
+__device__ __forceinline__ void block_others(double (&yt)[1], const double (&p)[1], const double* c) {
+#define MXC_OTHERS1(ORDER, LAST, ROWS) MXC_OTHERS(MXC_UP1, ORDER, LAST, ROWS, [y] "+&v"(yt[0]), [p] "v"(p[0]))
+  if constexpr (!UP) {
+    if constexpr (B == 0) MXC_OTHERS1(MXC_ASC, 15, "0xe");
+    if constexpr (B == 1) MXC_OTHERS1(MXC_ASC, 15, "0xc");
+    if constexpr (B == 2) MXC_OTHERS1(MXC_ASC, 15, "0x8");
+  } else {
+    if constexpr (B == 3) MXC_OTHERS1(MXC_DESC, 0, "0x7");
+    if constexpr (B == 2) MXC_OTHERS1(MXC_DESC, 0, "0x3");
+    if constexpr (B == 1) MXC_OTHERS1(MXC_DESC, 0, "0x1");
+  }
+}
+#define MXC_PAIR [y] "+&v"(yt[0]), [z] "+&v"(yt[1])
+template <int B, bool UP>
+__device__ __forceinline__ void block_others(double (&yt)[2], const double (&p)[2], const double* c) {
+#define MXC_OTHERS2(ORDER, LAST, ROWS) \
+  asm volatile("s_nop 1\n\t" ORDER(MXC_UP2, "", ROWS) MXC_UP2("", LAST, ROWS) "s_nop 1" \
+               : MXC_PAIR : [p] "v"(p[0]), [q] "v"(p[1]), MXC_COLUMNS)
+  if constexpr (!UP) {
+    if constexpr (B == 0) MXC_OTHERS2(MXC_ASC, 15, "0xe");
+    if constexpr (B == 1) MXC_OTHERS2(MXC_ASC, 15, "0xc");
+    if constexpr (B == 2) MXC_OTHERS2(MXC_ASC, 15, "0x8");
+  } else {
+    if constexpr (B == 3) MXC_OTHERS2(MXC_DESC, 0, "0x7");
+    if constexpr (B == 2) MXC_OTHERS2(MXC_DESC, 0, "0x3");
+    if constexpr (B == 1) MXC_OTHERS2(MXC_DESC, 0, "0x1");
+  }
+}
+
+template <int B, bool UP, int NV>
+__device__ __forceinline__ void block_solve(double (&yt)[NV], const double (&c)[NT], double* xw, int lane) {
+  block_own<B, UP>(yt, c + 16 * B);
+  if constexpr (UP ? B > 0 : B < 3) {
+    double p[NV];
 #pragma unroll
-      for (int v = 0; v < NV; v++) yl[v] = fma(-uk, readlane(yl[v] * dl, k), yl[v]);
-    }
+    for (int v = 0; v < NV; v++) xw[v * WAVE + lane] = yt[v];
+    wave_sync();
 #pragma unroll
-    for (int v = 0; v < NV; v++) yl[v] *= dl;
+    for (int v = 0; v < NV; v++) p[v] = xw[v * WAVE + 16 * B + (lane & 15)];
+    wave_sync();
+    block_others<B, UP>(yt, p, c + 16 * B);
   }
 }
 
 template <int NV>
+__device__ __forceinline__ void solve_blocks(double (&yt)[NV], const double (&c)[NT], double dt, double* ws, int lane) {
+  double* xw = ws + L_UNION;  // free between the right-hand sides
+  block_solve<0, false>(yt, c, xw, lane);
+  block_solve<1, false>(yt, c, xw, lane);
+  block_solve<2, false>(yt, c, xw, lane);
+  block_solve<3, false>(yt, c, xw, lane);
+  block_solve<3, true>(yt, c, xw, lane);
+  block_solve<2, true>(yt, c, xw, lane);
+  block_solve<1, true>(yt, c, xw, lane);
+  block_solve<0, true>(yt, c, xw, lane);
+#pragma unroll
+  for (int v = 0; v < NV; v++) yt[v] *= dt;
+}
+
+constexpr bool BLOCK_SOLVES = LU_2D && NT == WAVE;  // a try's factors then have 0 on c's diagonal (lu_factor)
+
+// BLOCKS: c has 0 on its diagonal (BLOCK_SOLVES)
+template <int NV, bool BLOCKS = false>
 __device__ __forceinline__ void solve(double (&yl)[NV], double (&yt)[NV], const double (&c)[NT], const LeadRow& a21,
                                       double dl, double dt, double* ws, int lane) {
-  ws = opaque_lds(ws);
   lane = opaque_lane(lane);
+  ws = opaque_lds(ws);
   solve_lead_forward(yl, yt, a21, ws, lane);
-  solve_trailing(yt, c, dt, lane);
+  if constexpr (BLOCKS)
+    solve_blocks(yt, c, dt, ws, lane);
+  else
+    solve_trailing(yt, c, dt, lane);
+  if constexpr (K0 > 0) {  // a rounded product here, not contracted into the sums that follow
+#pragma unroll
+    for (int v = 0; v < NV; v++) pin(yt[v]);
+  }
   solve_lead_backward(yl, yt, dl, ws, lane);
 }
 

@@ -270,7 +270,7 @@ __device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, do
 __device__ __forceinline__ void w_solve(double& yl, double& yt, const double (&c)[NT], const LeadRow& a21,
                                         const StageKeep& kp, double dtr, double* ws, int lane) {
   double vl[1] = {yl}, vt[1] = {yt};
-  solve<1>(vl, vt, c, a21, kp.dl, dtr, ws, lane);
+  solve<1, BLOCK_SOLVES>(vl, vt, c, a21, kp.dl, dtr, ws, lane);
   const double sk = vsum(vl[0], vt[0], lane) * kp.c0;
   yl = vl[0] + sk * kp.Ul;
   yt = vt[0] + sk * kp.Ut;

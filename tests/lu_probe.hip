@@ -2,7 +2,8 @@
 // matrix, row-major, elimination order. out: per layout, the factors [NS][NS] as the solves take them (unit L below the
 // diagonal, U of the lead rows, U' of the trailing block), then 1 / U_ii [NS]. One workgroup of one wavefront.
 
-extern "C" __global__ void __launch_bounds__(WAVE) mxc_lu_probe(const double* __restrict__ W, double* __restrict__ out) {
+extern "C" __global__ void __launch_bounds__(WAVE) mxc_lu_probe(const double* __restrict__ W, const double* __restrict__ b,
+                                                                     double* __restrict__ out) {
   extern __shared__ double lds[];
   const int lane = (int)threadIdx.x;
 #pragma unroll 1
@@ -21,7 +22,7 @@ extern "C" __global__ void __launch_bounds__(WAVE) mxc_lu_probe(const double* __
     else
       factor_rows(c, a21, dl, dt, lds, lane);
     wave_sync();
-    double* o = out + which * (NS * NS + NS);
+    double* o = out + which * (NS * NS + 4 * NS);
     for (int e = lane; e < K0 * NS; e += WAVE) o[e] = lds[e];
     if (lane < NT) {
 #pragma unroll
@@ -31,6 +32,31 @@ extern "C" __global__ void __launch_bounds__(WAVE) mxc_lu_probe(const double* __
     }
     if (lane < K0) o[NS * NS + lane] = dl;
     if (lane < NT) o[NS * NS + K0 + lane] = dt;
+    wave_sync();
+    double y1l[1], y1t[1], y2l[2], y2t[2];
+    auto get = [&](int v, double& yl, double& yt) {
+      yl = lane < K0 ? b[v * NS + lane] : 0.0;
+      yt = lane < NT ? b[v * NS + K0 + lane] : 0.0;
+    };
+    get(0, y1l[0], y1t[0]);
+    get(1, y2l[0], y2t[0]);
+    get(2, y2l[1], y2t[1]);
+    if (which == 0 && BLOCK_SOLVES) {
+#pragma unroll
+      for (int j = 0; j < NT; j++) c[j] = j == lane ? 0.0 : c[j];
+      solve<1, BLOCK_SOLVES>(y1l, y1t, c, a21, dl, dt, lds, lane);
+      solve<2, BLOCK_SOLVES>(y2l, y2t, c, a21, dl, dt, lds, lane);
+    } else {
+      solve<1>(y1l, y1t, c, a21, dl, dt, lds, lane);
+      solve<2>(y2l, y2t, c, a21, dl, dt, lds, lane);
+    }
+    auto put = [&](int v, double yl, double yt) {
+      if (lane < K0) o[NS * NS + (1 + v) * NS + lane] = yl;
+      if (lane < NT) o[NS * NS + (1 + v) * NS + K0 + lane] = yt;
+    };
+    put(0, y1l[0], y1t[0]);
+    put(1, y2l[0], y2t[0]);
+    put(2, y2l[1], y2t[1]);
     wave_sync();
   }
 }

@@ -1,5 +1,5 @@
-"""The two-dimensional LU of M0 against the LU by rows: the same bits, at the edges of its slots (16 rows by 4 columns)
-and of the lead part (64 trailing rows), on random patterns (GPU)."""
+"""The two-dimensional LU of M0 against the LU by rows, and the solves by blocks against those by rows: the same bits, at
+the edges of the slots (16 rows by 4 columns) and of the lead part (64 trailing rows), on random patterns (GPU)."""
 
 import types
 from pathlib import Path
@@ -32,7 +32,7 @@ def network(species: int, seed: int):
 
 
 @pytest.mark.parametrize("species", [3, 16, 17, 63, 64, 65, 80, 81, 92])
-def test_both_layouts_give_the_same_factors(species):
+def test_both_layouts_give_the_same_factors_and_solutions(species):
     tab = _tables.build(network(species, species))
     assert _kernels.lu_layout(tab)["use"] and tab.k0 == max(0, species - 64)
     src = (_kernels.header(tab, 1, 1e-6) + (_kernels.KERNEL_DIR / "common.hip").read_text() + PROBE.read_text())
@@ -45,9 +45,10 @@ def test_both_layouts_give_the_same_factors(species):
         W = np.where(tab.fill, rng.standard_normal((n, n)), 0.0) + 4.0 * np.eye(n)
         W = W * scale[0][:, None] * scale[1][None, :]
         w = torch.tensor(np.ascontiguousarray(W), device="cuda")
-        out = torch.full((2, n * n + n), float("nan"), dtype=torch.float64, device="cuda")
+        b = torch.tensor(scale[0] * rng.standard_normal((3, n)), device="cuda")
+        out = torch.full((2, n * n + 4 * n), float("nan"), dtype=torch.float64, device="cuda")
         _hip.launch(fn, 1, 64, 8 * tab.layout()["SIZE"], torch.cuda.current_stream().cuda_stream,
-                    [_hip.ptr(w), _hip.ptr(out)])  # fmt: skip
+                    [_hip.ptr(w), _hip.ptr(b), _hip.ptr(out)])  # fmt: skip
         torch.cuda.synchronize()
         got, want = out.cpu().numpy()
         assert np.isfinite(want).all()
