@@ -761,64 +761,94 @@ struct Pivot {
   static constexpr int M = (K < K0 ? 0 : LU_ML) + R / 16, S = R % 16, T = (K < K0 ? 0 : LU_TL) + R / 4, G = R % 4;
 };
 
+// Whether pivot K reaches row slot m below it, and column slot t right of it; in a dense matrix it reaches every one.
+template <bool DENSE>
+__device__ constexpr bool lu_row(int K, int m) { return DENSE || ((LU_ROWS[K] >> m) & 1u); }
+template <bool DENSE>
+__device__ constexpr bool lu_col(int K, int t) { return DENSE || ((LU_COLS[K] >> t) & 1u); }
+
 // Pivot K's multipliers -l_i K of this lane's rows (0 up to row K) from its column; lb: their exchange, [4][16 LU_M] in
 // LDS (each row of lanes writes its own part, the pivot's is read). The column itself keeps its unscaled entries.
-template <int K>
-__device__ __forceinline__ void lu_pivot(const LuBlock& A, double (&nl)[LU_M], double* lb, int lane) {
+// In a dense matrix, swap gathers the lanes that hold an entry below the pivot which the threshold rule would exchange
+// with it: |a_KK| not at least PIVTAU |a_iK|.
+template <int K, bool DENSE>
+__device__ __forceinline__ void lu_pivot(const LuBlock& A, double (&nl)[LU_M], double* lb, int lane, u64& swap) {
   using P = Pivot<K>;
-  const double dk = plain_rcp(readlane(A[P::M][P::T], 16 * P::G + P::S));
+  const double pivot = readlane(A[P::M][P::T], 16 * P::G + P::S);
+  const double dk = plain_rcp(pivot);
   const int s = opaque_lane(lane & 15);  // the step's mask made here
   double* mine = lb + (lane >> 4) * (16 * LU_M) + (lane & 15);
+  double top = 0.0;
 #pragma unroll
   for (int m = P::M; m < LU_M; m++)
-    if ((LU_ROWS[K] >> m) & 1u) {
+    if (lu_row<DENSE>(K, m)) {
       const double x = A[m][P::T] * dk;
-      mine[16 * m] = m > P::M || s > P::S ? x : 0.0;
+      const bool below = m > P::M || s > P::S;
+      mine[16 * m] = below ? x : 0.0;
+      if (DENSE) top = fmax(top, below ? fabs(A[m][P::T]) : 0.0);
     }
+  if (DENSE) swap |= __ballot(!(fabs(pivot) >= PIVTAU * top)) & (0xffffull << (16 * P::G));
   wave_sync();
 #pragma unroll
   for (int m = P::M; m < LU_M; m++)
-    if ((LU_ROWS[K] >> m) & 1u) nl[m] = -lb[P::G * (16 * LU_M) + 16 * m + (lane & 15)];
+    if (lu_row<DENSE>(K, m)) nl[m] = -lb[P::G * (16 * LU_M) + 16 * m + (lane & 15)];
   wave_sync();
 }
 
 // Pivot K's update of column slot t.
-template <int K>
+template <int K, bool DENSE>
 __device__ __forceinline__ void lu_update(LuBlock& A, const double (&nl)[LU_M], int t) {
   using P = Pivot<K>;
-  if (!((LU_COLS[K] >> t) & 1u)) return;
+  if (!lu_col<DENSE>(K, t)) return;
   const double u =
       t > P::T ? row_bcast<P::S>(A[P::M][t]) : row_bcast<P::S, (0xf << (P::G + 1)) & 0xf>(A[P::M][t]);
 #pragma unroll
   for (int m = P::M; m < LU_M; m++)
-    if ((LU_ROWS[K] >> m) & 1u) A[m][t] = fma(nl[m], u, A[m][t]);
+    if (lu_row<DENSE>(K, m)) A[m][t] = fma(nl[m], u, A[m][t]);
 }
 
 // Pivot K's updates, with pivot K + 1's multipliers (a chain of a broadcast, a reciprocal and an LDS round trip) taken
 // as soon as its own column is final, while the other columns are updated.
-template <int K>
-__device__ __forceinline__ void lu_step(LuBlock& A, double (&nl)[LU_M], double* lb, int lane) {
+template <int K, bool DENSE>
+__device__ __forceinline__ void lu_step(LuBlock& A, double (&nl)[LU_M], double* lb, int lane, u64& swap) {
   __builtin_amdgcn_sched_barrier(0);
   constexpr int TN = Pivot<K + 1 < NS ? K + 1 : K>::T;
   double next[LU_M];
   if constexpr (K + 1 < NS) {
-    lu_update<K>(A, nl, TN);
-    lu_pivot<K + 1>(A, next, lb, lane);
+    lu_update<K, DENSE>(A, nl, TN);
+    lu_pivot<K + 1, DENSE>(A, next, lb, lane, swap);
   }
 #pragma unroll
   for (int t = Pivot<K>::T; t < LU_T; t++)
-    if (t != TN) lu_update<K>(A, nl, t);
+    if (t != TN) lu_update<K, DENSE>(A, nl, t);
   if constexpr (K + 1 < NS) {
 #pragma unroll
     for (int m = 0; m < LU_M; m++) nl[m] = next[m];
   }
 }
 
-template <int... K>
-__device__ __forceinline__ void lu_steps(Seq<K...>, LuBlock& A, double* lb, int lane) {
+// Every pivot in turn; returns swap (0 but in a dense matrix).
+template <bool DENSE, int... K>
+__device__ __forceinline__ u64 lu_steps(Seq<K...>, LuBlock& A, double* lb, int lane) {
   double nl[LU_M];
-  lu_pivot<0>(A, nl, lb, lane);
-  (lu_step<K>(A, nl, lb, lane), ...);
+  u64 swap = 0;
+  lu_pivot<0, DENSE>(A, nl, lb, lane, swap);
+  (lu_step<K, DENSE>(A, nl, lb, lane, swap), ...);
+  return swap;
+}
+
+// The diagonal after the LU, by row slot: row s of a row slot has it in column slot s / 4 of the slot's four, in the
+// lanes of g = s % 4 (the other lanes' values are not the diagonal's).
+__device__ __forceinline__ void lu_diagonal(const LuBlock& A, double (&dg)[LU_M], int lane) {
+  const int q = (lane & 15) >> 2;
+#pragma unroll
+  for (int m = 0; m < LU_M; m++) {
+    const int t0 = m < LU_ML ? 4 * m : LU_TL + 4 * (m - LU_ML), last = m < LU_ML ? LU_TL : LU_T;
+    dg[m] = A[m][t0];
+#pragma unroll
+    for (int u = 1; u < 4; u++)
+      if (t0 + u < last) dg[m] = q == u ? A[m][t0 + u] : dg[m];
+  }
 }
 
 // A lane's place of slot (m, t) in a chunk of columns, column-major with LU_STRIDE doubles a column for the trailing
@@ -879,18 +909,10 @@ template <bool ZERO>
 __device__ __forceinline__ void lu_store(LuBlock& A, double (&c)[NT], LeadRow& a21, double& dl, double& dt, double* ws,
                                          int lane) {
   const LuPlace p(ws, lane);
-  const int s = lane & 15, g = lane >> 4, q = s >> 2;
+  const int s = lane & 15, g = lane >> 4;
   double* buf = ws + L_DV;
-  // the diagonal: row s of a row slot has it in column slot s / 4 of the slot's four, in the lanes of g = s % 4
   double dg[LU_M];
-#pragma unroll
-  for (int m = 0; m < LU_M; m++) {
-    const int t0 = m < LU_ML ? 4 * m : LU_TL + 4 * (m - LU_ML), last = m < LU_ML ? LU_TL : LU_T;
-    dg[m] = A[m][t0];
-#pragma unroll
-    for (int u = 1; u < 4; u++)
-      if (t0 + u < last) dg[m] = q == u ? A[m][t0 + u] : dg[m];
-  }
+  lu_diagonal(A, dg, lane);
   if (g == (s & 3)) {
 #pragma unroll
     for (int m = 0; m < LU_M; m++) buf[16 * m + s] = dg[m];
@@ -997,7 +1019,7 @@ __device__ __forceinline__ void lu_factor(LuBlock& A, double (&c)[NT], LeadRow& 
                                           int lane) {
   lane = opaque_lane(lane);
   ws = opaque_lds(ws);
-  lu_steps(Steps<NS>{}, A, ws + L_DV, lane);
+  lu_steps<false>(Steps<NS>{}, A, ws + L_DV, lane);
   wave_sync();
   lu_store<ZERO>(A, c, a21, dl, dt, opaque_lds(ws), opaque_lane(lane));
 }

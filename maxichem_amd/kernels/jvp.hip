@@ -781,9 +781,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
 #pragma unroll
           for (int j = 0; j < NT; j++) row[K0 + j] = (j == lane ? c[j] + igh : c[j]) - ut;
         }
-        if (lane == 0) *cmd = 1;
-        __syncthreads();
-        dense_lu(W, pr, dinv, lane, 0);
+        wave_sync();
+        dense_factor(W, pr, dinv, ws, cmd, lane);
         double K1l, K1t, K2l, K2t, K3l, K3t, K4l, K4t;
         to_lds(yv, Fl, Ft, lane);
         dense_solve(W, pr, dinv, yv, lane);

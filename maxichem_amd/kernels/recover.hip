@@ -102,13 +102,69 @@ __device__ void dense_lu(double* W, int* pr, double* dinv, int lane, int wv) {
   }
 }
 
+// The same factors by one wavefront in registers (common.hip's two-dimensional LU, every slot taken), where no pivot
+// exchanges rows; returns false and leaves W as it is where the threshold rule would exchange some. lb: the multipliers'
+// exchange. A try's W seldom exchanges (6 % of the tries of 367 recovered NCHO cells): this takes 33k cycles where
+// dense_lu takes 162k (its columns go through LDS and four barriers).
+__device__ __forceinline__ bool dense_lu_2d(double* W, int* pr, double* dinv, double* lb, int lane) {
+  lane = opaque_lane(lane);
+  const int s = lane & 15, g = lane >> 4;
+  LuBlock A;
+  auto row = [&](int m) { return (m < LU_ML ? 16 * m : K0 + 16 * (m - LU_ML)) + s; };
+  auto col = [&](int t) { return (t < LU_TL ? 4 * t : K0 + 4 * (t - LU_TL)) + g; };
+#pragma unroll
+  for (int m = 0; m < LU_M; m++) {
+    const int i = row(m);
+    const double* p = W + (NT == WAVE || i < NS ? i : NS - 1) * NS;  // rows past the matrix read its last one
+#pragma unroll
+    for (int t = 0; t < LU_T; t++) {
+      const double v = p[col(t)];  // a column past the matrix: the next row's, or a reciprocal's place
+      A[m][t] = lu_inside(m, t, lane) ? v : 0.0;
+    }
+  }
+  wave_sync();
+  if (lu_steps<true>(Steps<NS>{}, A, lb, lane) != 0ull) return false;
+  double dg[LU_M];
+  lu_diagonal(A, dg, lane);
+  if (g == (s & 3)) {
+#pragma unroll
+    for (int m = 0; m < LU_M; m++)
+      if (m < LU_ML ? row(m) < K0 : row(m) < NS) dinv[row(m)] = 1.0 / dg[m];
+  }
+  for (int i = lane; i < NS; i += WAVE) pr[i] = i;
+  wave_sync();
+#pragma unroll
+  for (int t = 0; t < LU_T; t++) {
+    const int j = col(t);
+    const double d = dinv[j < NS ? j : NS - 1];
+#pragma unroll
+    for (int m = 0; m < LU_M; m++) {
+      const int i = row(m);
+      if (lu_inside(m, t, lane)) W[i * NS + j] = i > j ? A[m][t] * d : A[m][t];
+    }
+  }
+  wave_sync();
+  return true;
+}
+
+// W's factors for the workgroup's first wavefront: in its registers, or with the other wavefronts (cmd calls them).
+__device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane) {
+  if constexpr (LU_2D) {
+    if (dense_lu_2d(W, pr, dinv, ws + L_DV, lane)) return;
+  }
+  if (lane == 0) *cmd = 1;
+  __syncthreads();
+  dense_lu(W, pr, dinv, lane, 0);
+}
+
 // y <- W^-1 y with dense_lu's factors; y is the vector in LDS (elimination order). Up to ROW_REGISTERS species, this
 // lane's row of the factors (row lane, clamped in bounds) is loaded into registers before the substitutions, so the
 // chain from step to step is a readlane and an fma with no LDS wait (beyond that the row would not fit the
-// registers, and its entries are read in the steps). Rows WAVE and beyond (a second row per lane) read their entries
-// in the steps. Every update is kept by a select, as the substitutions' order fixes the bits.
+// registers, and its entries are read in the steps). Rows WAVE and beyond (a second row per lane) read theirs
+// DENSE_BATCH steps at a time. Every update is kept by a select, as the substitutions' order fixes the bits.
 constexpr int ROW_REGISTERS = 80;
 constexpr bool ROW_IN_REGISTERS = NS <= ROW_REGISTERS;
+constexpr int DENSE_BATCH = 16;  // steps whose entries of a lane's second row are read together
 
 __device__ void dense_solve(const double* W, const int* pr, const double* dinv, double* y, int lane) {
   double a[2];
@@ -121,17 +177,45 @@ __device__ void dense_solve(const double* W, const int* pr, const double* dinv, 
     for (int k = 0; k < NS; k++) w0[k] = W[r0 * NS + k];
   }
   const double d0 = dinv[r0], d1 = dinv[r1];
+  // a batch of steps' entries of the second row, read for every lane (in bounds) so that no step waits on a branch
+  auto second = [&](double (&w)[DENSE_BATCH], int k0, int step) {
 #pragma unroll
-  for (int k = 0; k < NS - 1; k++) {
-    const double yk = readlane(k < WAVE ? a[0] : a[1], k & (WAVE - 1));
-    a[0] = lane > k ? fma(-(ROW_IN_REGISTERS ? w0[k] : W[r0 * NS + k]), yk, a[0]) : a[0];
-    if (NS > WAVE) a[1] = lane + WAVE > k && lane + WAVE < NS ? fma(-W[r1 * NS + k], yk, a[1]) : a[1];
+    for (int i = 0; i < DENSE_BATCH; i++)
+      if (NS > WAVE && k0 + i * step >= 0 && k0 + i * step < NS) w[i] = W[r1 * NS + k0 + i * step];
+  };
+#pragma unroll
+  for (int k0 = 0; k0 < NS - 1; k0 += DENSE_BATCH) {
+    double w1[DENSE_BATCH];
+    second(w1, k0, 1);
+#pragma unroll
+    for (int i = 0; i < DENSE_BATCH; i++) {
+      const int k = k0 + i;
+      if (k >= NS - 1) break;
+      const double yk = readlane(k < WAVE ? a[0] : a[1], k & (WAVE - 1));
+      const double u0 = fma(-(ROW_IN_REGISTERS ? w0[k] : W[r0 * NS + k]), yk, a[0]);
+      if (k < WAVE - 1) a[0] = lane > k ? u0 : a[0];
+      if (NS > WAVE) {
+        const double u1 = fma(-w1[i], yk, a[1]);
+        a[1] = lane + WAVE > k && lane + WAVE < NS ? u1 : a[1];
+      }
+    }
   }
 #pragma unroll
-  for (int k = NS - 1; k > 0; k--) {
-    const double zk = readlane(k < WAVE ? a[0] : a[1], k & (WAVE - 1)) * readlane(k < WAVE ? d0 : d1, k & (WAVE - 1));
-    a[0] = lane < k ? fma(-(ROW_IN_REGISTERS ? w0[k] : W[r0 * NS + k]), zk, a[0]) : a[0];
-    if (NS > WAVE) a[1] = lane + WAVE < k ? fma(-W[r1 * NS + k], zk, a[1]) : a[1];
+  for (int k1 = NS - 1; k1 > 0; k1 -= DENSE_BATCH) {
+    double w1[DENSE_BATCH];
+    second(w1, k1, -1);
+#pragma unroll
+    for (int i = 0; i < DENSE_BATCH; i++) {
+      const int k = k1 - i;
+      if (k <= 0) break;
+      const double zk = readlane(k < WAVE ? a[0] * d0 : a[1] * d1, k & (WAVE - 1));
+      const double u0 = fma(-(ROW_IN_REGISTERS ? w0[k] : W[r0 * NS + k]), zk, a[0]);
+      a[0] = lane < k ? u0 : a[0];
+      if (NS > WAVE && k > WAVE) {
+        const double u1 = fma(-w1[i], zk, a[1]);
+        a[1] = lane + WAVE < k ? u1 : a[1];
+      }
+    }
   }
   wave_sync();
   if (lane < NS) y[lane] = a[0] * d0;
@@ -221,9 +305,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
 #pragma unroll
           for (int j = 0; j < NT; j++) row[K0 + j] = (j == lane ? c[j] + igh : c[j]) - ut;
         }
-        if (lane == 0) *cmd = 1;
-        __syncthreads();
-        dense_lu(W, pr, dinv, lane, 0);
+        wave_sync();
+        dense_factor(W, pr, dinv, ws, cmd, lane);
         double K1l, K1t, K2l, K2t, K3l, K3t, K4l, K4t;
         to_lds(yv, Fl, Ft, lane);
         dense_solve(W, pr, dinv, yv, lane);

@@ -54,3 +54,49 @@ def test_both_layouts_give_the_same_factors_and_solutions(species):
         assert np.isfinite(want).all()
         assert np.array_equal(got, want)
     module.unload()
+
+
+@pytest.mark.parametrize("stem", ["synthetic", "NCHO"])
+def test_the_register_lu_takes_the_matrices_without_exchanges(read_network, stem):
+    # the recovery's fast LU gives dense_lu's factors bit for bit where the threshold rule exchanges no row, and leaves
+    # every other matrix, and one with a NaN, as it is
+    import helpers
+    from probes import Probes
+
+    from maxichem_amd import standin
+
+    net = standin.load(stem) if stem == "NCHO" else read_network(stem)
+    probes = Probes(net)
+    tab = probes.tab
+    n = tab.ns
+    rng = np.random.default_rng(5)
+    mats = [rng.standard_normal((n, n)) + d * np.eye(n) for d in (4.0 * n, 2.0 * n, n, 3.0, 0.5) for _ in range(3)]
+    edge = 10.0 * np.eye(n)
+    edge[1:, 0] = 100.0  # |W_00| is PIVTAU times the column's largest: kept; a bit more exchanges
+    more = edge.copy()
+    more[n - 1, 0] = np.nextafter(100.0, 200.0)
+    nan = mats[0].copy()
+    nan[n - 1, 3] = np.nan
+    mats = [*mats, edge, more, np.eye(n), *helpers.adversarial_matrices(n, rng), nan]
+    want, rows, dinv, _ = probes.run_dense(np.array(mats), np.zeros((len(mats), n)))
+    src = (_kernels.header(tab, 1, 1e-6) + "".join((_kernels.KERNEL_DIR / f).read_text()
+           for f in ("common.hip", "guard.hip", "recover.hip")) + PROBE.with_name("dense_2d_probe.hip").read_text())  # fmt: skip
+    module = _hip.Module(_hip.compile_source(src, "dense_2d_probe.hip"), torch.cuda.current_device())
+    W = torch.tensor(np.array(mats), device="cuda")
+    d = torch.zeros(len(mats), n, dtype=torch.float64, device="cuda")
+    took = torch.zeros(len(mats), dtype=torch.int32, device="cuda")
+    lds = 8 * (tab.layout()["SIZE"] + n * n + 2 * n) + 4 * n
+    _hip.launch(module.function("mxc_dense_2d_probe"), len(mats), 64, lds, torch.cuda.current_stream().cuda_stream,
+                [_hip.ptr(W), _hip.ptr(d), _hip.ptr(took)])  # fmt: skip
+    torch.cuda.synchronize()
+    got, d, took = W.cpu().numpy(), d.cpu().numpy(), took.cpu().numpy()
+    kept = [list(r) == list(range(n)) for r in rows]
+    assert kept[:3] == [True] * 3 and took[15] == 1 and took[16] == 0 and sum(took) < len(mats)
+    for m, a in enumerate(mats):
+        assert bool(took[m]) == (kept[m] and bool(np.isfinite(a).all())), m
+        if took[m]:
+            assert np.array_equal(got[m], want[m]) and np.array_equal(d[m], dinv[m])
+        else:
+            assert np.array_equal(got[m], a, equal_nan=True)
+    module.unload()
+    probes.close()
