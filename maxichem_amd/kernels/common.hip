@@ -148,12 +148,6 @@ __device__ __forceinline__ void tie(float& a, float b) { asm volatile("" : "+v"(
 
 __device__ __forceinline__ bool wave_all(bool p) { return __ballot(!p) == 0ull; }
 
-// A stream word's coefficient: +-1 or +-2 from its sign and x2 bits.
-__device__ __forceinline__ double coefficient(u32 w, int neg, int dbl) {
-  const double c = ((w >> dbl) & 1u) ? 2.0 : 1.0;
-  return ((w >> neg) & 1u) ? -c : c;
-}
-
 // A stream word's term: d times the word's coefficient, exactly as fma(coefficient, d, .) takes it: x2 is an exponent
 // step, and the sign (the word's bit 31) is XORed into the double's sign bit, or put there where d is not SIGNED (then
 // one instruction). No compares and selects, and no wait states for condition masks.

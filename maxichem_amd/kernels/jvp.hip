@@ -164,7 +164,29 @@ template <bool HD>
 __device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, double Yet, double Kl, double Kt, double& Fel,
                             double& Fet, double& Fedl, double& Fedt, NetP net, double nd, double ndd,
                             double* ts, const double* rk, const double* rkd, int lane) {
+  lane = opaque_lane(lane);
   const bool hl = lane < K0, ht = lane < NT;
+  // every table word and rate coefficient (and its tangent) the rounds and the S v stream need, loaded first: they
+  // arrive while n is made (in bounds: the last round's spare lanes read reaction NR - 1, and store nothing)
+  net = opaque(net);
+  const gptr<u64> rxe = net->rxe;
+  const gptr<u32> svw = net->svw;
+  const gptr<u32> rowp = net->rowp;
+  const u32 rpl = rowp[hl ? lane : 0], rpt = rowp[K0 + (ht ? lane : 0)];
+  u64 wr[RROUNDS];
+  double rf[RROUNDS], rr[RROUNDS], rfd[RROUNDS], rrd[RROUNDS];
+  u32 wb[SV_ROUNDS];
+#pragma unroll
+  for (int q = 0; q < RROUNDS; q++) {
+    const int r = q * WAVE + lane < NR ? q * WAVE + lane : NR - 1;
+    wr[q] = rxe[r];
+    rf[q] = rk[r];
+    rr[q] = rk[NR + r];
+    rfd[q] = rkd[r];
+    rrd[q] = rkd[NR + r];
+  }
+#pragma unroll
+  for (int q = 0; q < SV_ROUNDS; q++) wb[q] = svw[q * WAVE + lane];
   double sums[3] = {(hl ? Yl : 0.0) + (ht ? Yt : 0.0), (hl ? Yel : 0.0) + (ht ? Yet : 0.0),
                     HD ? (hl ? Kl : 0.0) + (ht ? Kt : 0.0) : 0.0};
   wave_sums(sums);
@@ -188,81 +210,70 @@ __device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, do
     n[NS] = 1.0;
     n[SN + NS] = n[2 * SN + NS] = n[3 * SN + NS] = 0.0;
   }
+  double* part = ts + J_PART;  // [4][NPART]
+#pragma unroll
+  for (int i = 0; i < 4 * NPART; i += WAVE)
+    if (i + lane < 4 * NPART) part[i + lane] = 0.0;
   wave_sync();
-  net = opaque(net);
-  const gptr<u64> rxe = net->rxe;
-  const gptr<u32> svw = net->svw;
-  const gptr<u32> rowp = net->rowp;
   double* V = ts + J_V;  // [4][NR + 1]
   constexpr int SV = NR + 1;
   auto nh = [&](int i) { return Hyper{n[i], n[SN + i], HD ? n[2 * SN + i] : 0.0, HD ? n[3 * SN + i] : 0.0}; };
-  // every round's reaction word loaded first (in bounds: the last round's spare lanes read reaction NR - 1), so the
-  // rounds wait for one memory latency, not one each
-  u64 wr[RROUNDS];
-#pragma unroll
-  for (int q = 0; q < RROUNDS; q++) wr[q] = rxe[q * WAVE + lane < NR ? q * WAVE + lane : NR - 1];
 #pragma unroll
   for (int q = 0; q < RROUNDS; q++) {
     const int r = q * WAVE + lane;
-    if (r >= NR) break;
     const u64 w = wr[q];
     const Hyper pf = hmul(hmul(nh(species_of(w, 0)), nh(species_of(w, 1))), nh(species_of(w, 2)));
     const Hyper pr = hmul(hmul(nh(species_of(w, 3)), nh(species_of(w, 4))), nh(species_of(w, 5)));
-    const Hyper vf = hmul(Hyper{rk[r], rkd[r], 0.0, 0.0}, pf);
-    const Hyper vr = hmul(Hyper{rk[NR + r], rkd[NR + r], 0.0, 0.0}, pr);
-    V[r] = vf.v - vr.v;
-    V[SV + r] = vf.e - vr.e;
-    V[2 * SV + r] = vf.d - vr.d;
-    V[3 * SV + r] = vf.ed - vr.ed;
+    const Hyper vf = hmul(Hyper{rf[q], rfd[q], 0.0, 0.0}, pf);
+    const Hyper vr = hmul(Hyper{rr[q], rrd[q], 0.0, 0.0}, pr);
+    const int at = r < NR ? r : NR;  // the last round's spare lanes write the padding term, set to 0 after them
+    V[at] = vf.v - vr.v;
+    V[SV + at] = vf.e - vr.e;
+    V[2 * SV + at] = vf.d - vr.d;
+    V[3 * SV + at] = vf.ed - vr.ed;
   }
   if (lane == 0) V[NR] = V[SV + NR] = V[2 * SV + NR] = V[3 * SV + NR] = 0.0;
   wave_sync();
-  // S v by the rhs's lane streams, four parts at once
-  double* part = ts + J_PART;  // [4][NPART]
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  // the words of TB rounds loaded together, ahead of their terms (one memory latency per batch; a batch of 16 would
-  // make the tangent kernel spill)
-  constexpr int TB = 8;
-#pragma unroll 1
-  for (int q0 = 0; q0 < SV_ROUNDS; q0 += TB) {
-    u32 wb[TB];
+  // S v by the rhs's lane streams, four parts at once, each added at its piece (as stream_sum)
 #pragma unroll
-    for (int i = 0; i < TB; i++) wb[i] = q0 + i < SV_ROUNDS ? svw[(q0 + i) * WAVE + lane] : (u32)NR;
+  for (int q = 0; q < SV_ROUNDS; q++) {
+    const u32 w = wb[q];
+    const int r = (int)(w & SV_R_MASK), piece = (int)((w >> SV_PIECE) & SV_PIECE_MASK);
+    // the word's +-1 or +-2: a product with it is exact
+    const double c = __longlong_as_double(
+        (long long)(u64)((w & 0x80000000u) | (0x3ff00000u + (((w >> SV_DBL) & 1u) << 20))) << 32);
 #pragma unroll
-    for (int i = 0; i < TB; i++) {
-      const u32 w = wb[i];
-      const int r = (int)(w & SV_R_MASK);
-      const double c = coefficient(w, SV_NEG, SV_DBL);
-#pragma unroll
-      for (int p = 0; p < 4; p++) acc[p] = fma(c, V[p * SV + r], acc[p]);
-      if ((w >> SV_END) & 1u) {
-        const int piece = (int)((w >> SV_PIECE) & SV_PIECE_MASK);
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-          part[p * NPART + piece] = acc[p];
-          acc[p] = 0.0;
-        }
-      }
-    }
+    for (int p = 0; p < 4; p++) lds_add(part + p * NPART + piece, c * V[p * SV + r]);
   }
   wave_sync();
   // F = (ntot / nd) S v in hyper-duals
   const double ind = 1.0 / nd;
   const Hyper ixf = hmul(Hyper{nt, nte, ntd, 0.0}, Hyper{ind, -ndd * ind * ind, 0.0, 0.0});
-  auto row = [&](int k, double& fe, double& fed) {
-    const u32 rp = rowp[k];
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int e = 0; e < (int)(rp >> 16); e++) {
+  auto row = [&](u32 rp, double& fe, double& fed) {
+    const int first = (int)(rp & 0xffffu), count = (int)(rp >> 16);
+    double v[PIECE_MAX][4], s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int p = 0; p < 4; p++) s[p] += part[p * NPART + (rp & 0xffffu) + e];
-    }
+    for (int e = 0; e < PIECE_MAX; e++)
+#pragma unroll
+      for (int p = 0; p < 4; p++) v[e][p] = part[p * NPART + (e < count ? first + e : 0)];
+#pragma unroll
+    for (int e = 0; e < PIECE_MAX; e++)
+#pragma unroll
+      for (int p = 0; p < 4; p++) s[p] = e < count ? s[p] + v[e][p] : s[p];
     const Hyper F = hmul(ixf, Hyper{s[0], s[1], s[2], s[3]});
     fe = F.e;
     fed = F.ed;
   };
   Fel = Fet = Fedl = Fedt = 0.0;
-  if (hl) row(lane, Fel, Fedl);
-  if (ht) row(K0 + lane, Fet, Fedt);
+  double fe, fed;
+  if (K0 > 0) {
+    row(rpl, fe, fed);
+    Fel = hl ? fe : 0.0;
+    Fedl = hl ? fed : 0.0;
+  }
+  row(rpt, fe, fed);
+  Fet = ht ? fe : 0.0;
+  Fedt = ht ? fed : 0.0;
   wave_sync();
 }
 
