@@ -148,22 +148,51 @@ __device__ __forceinline__ void rates_tangent(double* ts, double* rkd, double T,
 
 // ---- F in hyper-dual numbers ----
 
-// A hyper-dual number: value, eps part, del part, eps-del part.
+// A hyper-dual number with ND del directions: value, eps part, then each direction's del and eps-del parts.
+template <int ND>
 struct Hyper {
-  double v, e, d, ed;
+  double v, e, d[ND ? ND : 1], ed[ND ? ND : 1];
 };
-__device__ __forceinline__ Hyper hmul(Hyper a, Hyper b) {
-  return {a.v * b.v, fma(a.e, b.v, a.v * b.e), fma(a.d, b.v, a.v * b.d),
-          fma(a.ed, b.v, fma(a.e, b.d, fma(a.d, b.e, a.v * b.ed)))};
+template <int ND>
+__device__ __forceinline__ Hyper<ND> hyper(double v, double e, double d = 0.0) {
+  Hyper<ND> h;
+  h.v = v;
+  h.e = e;
+#pragma unroll
+  for (int i = 0; i < (ND ? ND : 1); i++) h.d[i] = d, h.ed[i] = 0.0;
+  return h;
+}
+template <int ND>
+__device__ __forceinline__ Hyper<ND> hmul(const Hyper<ND>& a, const Hyper<ND>& b) {
+  Hyper<ND> r;
+  r.v = a.v * b.v;
+  r.e = fma(a.e, b.v, a.v * b.e);
+#pragma unroll
+  for (int i = 0; i < ND; i++) {
+    r.d[i] = fma(a.d[i], b.v, a.v * b.d[i]);
+    r.ed[i] = fma(a.ed[i], b.v, fma(a.e, b.d[i], fma(a.d[i], b.e, a.v * b.ed[i])));
+  }
+  return r;
 }
 
-// The eps part (Fe) of F(Y + eps Ye; rates + eps ratesdot, nd + eps ndd) and, with HD, the eps-del part (Fed) of
-// F(Y + eps Ye + del K; ...): lead / trailing parts per lane. Uses the tangent region ts (n, v and pieces, four parts
-// each) and the call's rate coefficients rk and their tangents rkd.
-template <bool HD>
-__device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, double Yet, double Kl, double Kt, double& Fel,
-                            double& Fet, double& Fedl, double& Fedt, NetP net, double nd, double ndd,
-                            double* ts, const double* rk, const double* rkd, int lane) {
+// Two del directions at once, where the parts of the second fit the LDS that a try's dv terms leave free after its
+// factorization: value and eps parts, and each stream word, then serve both.
+constexpr int HD_PARTS = NS + 1 + NR + 1 + NPART;  // doubles of one part: n, v and the pieces
+constexpr int HD = 2 * HD_PARTS <= L_SPARE + WAVE - L_DV ? 2 : 1;
+
+// The eps part (Fel, Fet) of F(Y + eps Ye; rates + eps ratesdot, nd + eps ndd) and, per del direction i < ND, the
+// eps-del part (Gl[i], Gt[i]) of F(Y + eps Ye + del K_i; ...): lead / trailing parts per lane. Uses the tangent region
+// ts (n, v and pieces, four parts each), spare (the cell's dv terms' place, for the parts after the fourth) and the
+// call's rate coefficients rk and their tangents rkd. What bounds it is the LDS: the gathers of n and of the stream's
+// terms, and the adds (cycles of one wavefront, NCHO, a try's six evaluations of F: 166k waiting for each round's
+// global reads, 124k with those ahead, 85k with two directions at once and no del parts where none are asked for).
+template <int ND>
+__device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, double Yet, const double (&Kl)[ND ? ND : 1],
+                                            const double (&Kt)[ND ? ND : 1], double& Fel, double& Fet,
+                                            double (&Gl)[ND ? ND : 1], double (&Gt)[ND ? ND : 1], NetP net, double nd,
+                                            double ndd, double* ts, double* spare, const double* rk, const double* rkd,
+                                            int lane) {
+  constexpr int P = 2 + 2 * ND, SN = NS + 1, SV = NR + 1;  // parts: v, e, then each direction's d, ed
   lane = opaque_lane(lane);
   const bool hl = lane < K0, ht = lane < NT;
   // every table word and rate coefficient (and its tangent) the rounds and the S v stream need, loaded first: they
@@ -187,54 +216,78 @@ __device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, do
   }
 #pragma unroll
   for (int q = 0; q < SV_ROUNDS; q++) wb[q] = svw[q * WAVE + lane];
-  double sums[3] = {(hl ? Yl : 0.0) + (ht ? Yt : 0.0), (hl ? Yel : 0.0) + (ht ? Yet : 0.0),
-                    HD ? (hl ? Kl : 0.0) + (ht ? Kt : 0.0) : 0.0};
-  wave_sums(sums);
-  const double nt = sums[0], nte = sums[1], ntd = sums[2];
-  // x = nd / ntot in hyper-duals: nd has an eps part, 1 / ntot all four
-  const double in = 1.0 / nt;
-  const Hyper inv{in, -nte * in * in, -ntd * in * in, 2.0 * nte * ntd * in * in * in};
-  const Hyper xf = hmul(Hyper{nd, ndd, 0.0, 0.0}, inv);
-  double* n = ts + J_N;  // [4][NS + 1]
-  constexpr int SN = NS + 1;
-  auto put = [&](int i, double y, double ye, double kd) {
-    const Hyper v = hmul(xf, Hyper{y, ye, kd, 0.0});
-    n[i] = v.v;
-    n[SN + i] = v.e;
-    n[2 * SN + i] = v.d;
-    n[3 * SN + i] = v.ed;
-  };
-  if (hl) put(lane, Yl, Yel, HD ? Kl : 0.0);
-  if (ht) put(K0 + lane, Yt, Yet, HD ? Kt : 0.0);
-  if (lane == 0) {
-    n[NS] = 1.0;
-    n[SN + NS] = n[2 * SN + NS] = n[3 * SN + NS] = 0.0;
-  }
-  double* part = ts + J_PART;  // [4][NPART]
+  auto np = [&](int p) { return p < 4 ? ts + J_N + p * SN : spare + (p - 4) * SN; };
+  auto vp = [&](int p) { return p < 4 ? ts + J_V + p * SV : spare + 2 * SN + (p - 4) * SV; };
+  auto pp = [&](int p) { return p < 4 ? ts + J_PART + p * NPART : spare + 2 * (SN + SV) + (p - 4) * NPART; };
+  double sums[2 + ND];
+  sums[0] = (hl ? Yl : 0.0) + (ht ? Yt : 0.0);
+  sums[1] = (hl ? Yel : 0.0) + (ht ? Yet : 0.0);
 #pragma unroll
-  for (int i = 0; i < 4 * NPART; i += WAVE)
-    if (i + lane < 4 * NPART) part[i + lane] = 0.0;
+  for (int i = 0; i < ND; i++) sums[2 + i] = (hl ? Kl[i] : 0.0) + (ht ? Kt[i] : 0.0);
+  wave_sums(sums);
+  const double nt = sums[0], nte = sums[1];
+  // x = nd / ntot in hyper-duals: nd has an eps part, 1 / ntot all of them
+  const double in = 1.0 / nt;
+  Hyper<ND> inv = hyper<ND>(in, -nte * in * in), nth = hyper<ND>(nt, nte);
+#pragma unroll
+  for (int i = 0; i < ND; i++) {
+    const double ntd = sums[2 + i];
+    inv.d[i] = -ntd * in * in;
+    inv.ed[i] = 2.0 * nte * ntd * in * in * in;
+    nth.d[i] = ntd;
+  }
+  const Hyper<ND> xf = hmul(hyper<ND>(nd, ndd), inv);
+  auto put = [&](int i, double y, double ye, const double (&k)[ND ? ND : 1]) {
+    Hyper<ND> h = hyper<ND>(y, ye);
+#pragma unroll
+    for (int j = 0; j < ND; j++) h.d[j] = k[j];
+    h = hmul(xf, h);
+    np(0)[i] = h.v;
+    np(1)[i] = h.e;
+#pragma unroll
+    for (int j = 0; j < ND; j++) np(2 + 2 * j)[i] = h.d[j], np(3 + 2 * j)[i] = h.ed[j];
+  };
+  if (hl) put(lane, Yl, Yel, Kl);
+  if (ht) put(K0 + lane, Yt, Yet, Kt);
+  if (lane == 0) {
+    np(0)[NS] = 1.0;
+#pragma unroll
+    for (int p = 1; p < P; p++) np(p)[NS] = 0.0;
+  }
+#pragma unroll
+  for (int p = 0; p < P; p++)
+#pragma unroll
+    for (int i = 0; i < NPART; i += WAVE)
+      if (i + lane < NPART) pp(p)[i + lane] = 0.0;
   wave_sync();
-  double* V = ts + J_V;  // [4][NR + 1]
-  constexpr int SV = NR + 1;
-  auto nh = [&](int i) { return Hyper{n[i], n[SN + i], HD ? n[2 * SN + i] : 0.0, HD ? n[3 * SN + i] : 0.0}; };
+  auto nh = [&](int i) {
+    Hyper<ND> h;
+    h.v = np(0)[i];
+    h.e = np(1)[i];
+#pragma unroll
+    for (int j = 0; j < ND; j++) h.d[j] = np(2 + 2 * j)[i], h.ed[j] = np(3 + 2 * j)[i];
+    return h;
+  };
 #pragma unroll
   for (int q = 0; q < RROUNDS; q++) {
     const int r = q * WAVE + lane;
     const u64 w = wr[q];
-    const Hyper pf = hmul(hmul(nh(species_of(w, 0)), nh(species_of(w, 1))), nh(species_of(w, 2)));
-    const Hyper pr = hmul(hmul(nh(species_of(w, 3)), nh(species_of(w, 4))), nh(species_of(w, 5)));
-    const Hyper vf = hmul(Hyper{rf[q], rfd[q], 0.0, 0.0}, pf);
-    const Hyper vr = hmul(Hyper{rr[q], rrd[q], 0.0, 0.0}, pr);
+    const Hyper<ND> pf = hmul(hmul(nh(species_of(w, 0)), nh(species_of(w, 1))), nh(species_of(w, 2)));
+    const Hyper<ND> pr = hmul(hmul(nh(species_of(w, 3)), nh(species_of(w, 4))), nh(species_of(w, 5)));
+    const Hyper<ND> vf = hmul(hyper<ND>(rf[q], rfd[q]), pf);
+    const Hyper<ND> vr = hmul(hyper<ND>(rr[q], rrd[q]), pr);
     const int at = r < NR ? r : NR;  // the last round's spare lanes write the padding term, set to 0 after them
-    V[at] = vf.v - vr.v;
-    V[SV + at] = vf.e - vr.e;
-    V[2 * SV + at] = vf.d - vr.d;
-    V[3 * SV + at] = vf.ed - vr.ed;
+    vp(0)[at] = vf.v - vr.v;
+    vp(1)[at] = vf.e - vr.e;
+#pragma unroll
+    for (int j = 0; j < ND; j++) vp(2 + 2 * j)[at] = vf.d[j] - vr.d[j], vp(3 + 2 * j)[at] = vf.ed[j] - vr.ed[j];
   }
-  if (lane == 0) V[NR] = V[SV + NR] = V[2 * SV + NR] = V[3 * SV + NR] = 0.0;
+  if (lane == 0) {
+#pragma unroll
+    for (int p = 0; p < P; p++) vp(p)[NR] = 0.0;
+  }
   wave_sync();
-  // S v by the rhs's lane streams, four parts at once, each added at its piece (as stream_sum)
+  // S v by the rhs's lane streams, every part at once, each added at its piece (as stream_sum)
 #pragma unroll
   for (int q = 0; q < SV_ROUNDS; q++) {
     const u32 w = wb[q];
@@ -243,38 +296,69 @@ __device__ __forceinline__ void rhs_tangent(double Yl, double Yt, double Yel, do
     const double c = __longlong_as_double(
         (long long)(u64)((w & 0x80000000u) | (0x3ff00000u + (((w >> SV_DBL) & 1u) << 20))) << 32);
 #pragma unroll
-    for (int p = 0; p < 4; p++) lds_add(part + p * NPART + piece, c * V[p * SV + r]);
+    for (int p = 0; p < P; p++) lds_add(pp(p) + piece, c * vp(p)[r]);
   }
   wave_sync();
   // F = (ntot / nd) S v in hyper-duals
   const double ind = 1.0 / nd;
-  const Hyper ixf = hmul(Hyper{nt, nte, ntd, 0.0}, Hyper{ind, -ndd * ind * ind, 0.0, 0.0});
-  auto row = [&](u32 rp, double& fe, double& fed) {
+  const Hyper<ND> ixf = hmul(nth, hyper<ND>(ind, -ndd * ind * ind));
+  auto row = [&](u32 rp) {
     const int first = (int)(rp & 0xffffu), count = (int)(rp >> 16);
-    double v[PIECE_MAX][4], s[4] = {0.0, 0.0, 0.0, 0.0};
+    double v[PIECE_MAX][P], s[P];
+#pragma unroll
+    for (int p = 0; p < P; p++) s[p] = 0.0;
 #pragma unroll
     for (int e = 0; e < PIECE_MAX; e++)
 #pragma unroll
-      for (int p = 0; p < 4; p++) v[e][p] = part[p * NPART + (e < count ? first + e : 0)];
+      for (int p = 0; p < P; p++) v[e][p] = pp(p)[e < count ? first + e : 0];
 #pragma unroll
     for (int e = 0; e < PIECE_MAX; e++)
 #pragma unroll
-      for (int p = 0; p < 4; p++) s[p] = e < count ? s[p] + v[e][p] : s[p];
-    const Hyper F = hmul(ixf, Hyper{s[0], s[1], s[2], s[3]});
-    fe = F.e;
-    fed = F.ed;
+      for (int p = 0; p < P; p++) s[p] = e < count ? s[p] + v[e][p] : s[p];
+    Hyper<ND> h = hyper<ND>(s[0], s[1]);
+#pragma unroll
+    for (int j = 0; j < ND; j++) h.d[j] = s[2 + 2 * j], h.ed[j] = s[3 + 2 * j];
+    return hmul(ixf, h);
   };
-  Fel = Fet = Fedl = Fedt = 0.0;
-  double fe, fed;
+  Fel = Fet = 0.0;
+#pragma unroll
+  for (int i = 0; i < (ND ? ND : 1); i++) Gl[i] = Gt[i] = 0.0;
   if (K0 > 0) {
-    row(rpl, fe, fed);
-    Fel = hl ? fe : 0.0;
-    Fedl = hl ? fed : 0.0;
+    const Hyper<ND> F = row(rpl);
+    Fel = hl ? F.e : 0.0;
+#pragma unroll
+    for (int i = 0; i < ND; i++) Gl[i] = hl ? F.ed[i] : 0.0;
   }
-  row(rpt, fe, fed);
-  Fet = ht ? fe : 0.0;
-  Fedt = ht ? fed : 0.0;
+  const Hyper<ND> F = row(rpt);
+  Fet = ht ? F.e : 0.0;
+#pragma unroll
+  for (int i = 0; i < ND; i++) Gt[i] = ht ? F.ed[i] : 0.0;
   wave_sync();
+}
+
+// Fdot(Y) alone: the eps part of F(Y + eps Ye; ...).
+__device__ __forceinline__ void rhs_eps(double Yl, double Yt, double Yel, double Yet, double& Fel, double& Fet, NetP net,
+                                        double nd, double ndd, double* ts, double* spare, const double* rk,
+                                        const double* rkd, int lane) {
+  const double none[1] = {0.0};
+  double gl[1], gt[1];
+  rhs_tangent<0>(Yl, Yt, Yel, Yet, none, none, Fel, Fet, gl, gt, net, nd, ndd, ts, spare, rk, rkd, lane);
+}
+
+// Fdot(N) and Jdot K_i for a try's four stages.
+__device__ __forceinline__ void stage_products(double Nl, double Nt, double Ndl, double Ndt, const double (&Kl)[4],
+                                               const double (&Kt)[4], double& Fel, double& Fet, double (&Gl)[4],
+                                               double (&Gt)[4], NetP net, double nd, double ndd, double* ts, double* spare,
+                                               const double* rk, const double* rkd, int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; i += HD) {
+    double kl[HD], kt[HD], gl[HD], gt[HD];
+#pragma unroll
+    for (int j = 0; j < HD; j++) kl[j] = Kl[i + j], kt[j] = Kt[i + j];
+    rhs_tangent<HD>(Nl, Nt, Ndl, Ndt, kl, kt, Fel, Fet, gl, gt, net, nd, ndd, ts, spare, rk, rkd, lane);
+#pragma unroll
+    for (int j = 0; j < HD; j++) Gl[i + j] = gl[j], Gt[i + j] = gt[j];
+  }
 }
 
 // W^-1 y (lead / trailing parts) with a try's factors: M0^-1 y, then the Sherman-Morrison term of w 1^T.
@@ -581,11 +665,13 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
         // the tangent of the try (every try under the adaptive contract: a rejected one sets the next step), with
         // its factors still in place
         const double ih = 1.0 / ha;
-        double Fel, Fet, Gl, Gt, Ql, Qt;  // Fdot(N); Jdot K_i (eps-del parts)
+        double Fel, Fet, Ql, Qt, Gl[4], Gt[4];  // Fdot(N), Fdot(Y); Jdot K_i (eps-del parts)
         double K1dl, K1dt, K2dl, K2dt, K3dl, K3dt, K4dl, K4dt;
-        rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K1l, K1t, Fel, Fet, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-        K1dl = Fel + Gl;
-        K1dt = Fet + Gt;
+        const double Kl[4] = {K1l, kp.K2l, K3l, K4l}, Kt[4] = {K1t, kp.K2t, K3t, K4t};
+        double* spare = ws + L_DV;
+        stage_products(Nl, Nt, Ndl, Ndt, Kl, Kt, Fel, Fet, Gl, Gt, net, nd, ndd, ts, spare, rk, rkd, lane);
+        K1dl = Fel + Gl[0];
+        K1dt = Fet + Gt[0];
         // adaptive: W = I / (gamma h) - J moves with h, W Kdot = bdot + Jdot K + hdot / (gamma h^2) K, and the stages'
         // K / h terms give -hdot / h^2 K
         const double sg = had * ih * ih / GAMMA, hq = had * ih * ih;
@@ -594,32 +680,28 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
           K1dt = fma(sg, K1t, K1dt);
         }
         w_solve(K1dl, K1dt, c, a21, kp, dtr, ws, lane);
-        rhs_tangent<true>(Nl, Nt, Ndl, Ndt, kp.K2l, kp.K2t, Ql, Qt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-        K2dl = fma(RODAS_C21 * ih, K1dl, Fel) + Gl;
-        K2dt = fma(RODAS_C21 * ih, K1dt, Fet) + Gt;
+        K2dl = fma(RODAS_C21 * ih, K1dl, Fel) + Gl[1];
+        K2dt = fma(RODAS_C21 * ih, K1dt, Fet) + Gt[1];
         if (ad) {
           K2dl += sg * kp.K2l - hq * RODAS_C21 * K1l;
           K2dt += sg * kp.K2t - hq * RODAS_C21 * K1t;
         }
         w_solve(K2dl, K2dt, c, a21, kp, dtr, ws, lane);
-        // stage 3: F at Y3 = N + 2 K1 along Ydot3 = Ndot + 2 Kdot1; Jdot K3 at N
-        double Y3el = Ndl + 2.0 * K1dl, Y3et = Ndt + 2.0 * K1dt, dummyl, dummyt;
-        rhs_tangent<false>(Nl + 2.0 * K1l, Nt + 2.0 * K1t, Y3el, Y3et, 0.0, 0.0, Ql, Qt, dummyl, dummyt, net, nd,
-                           ndd, ts, rk, rkd, lane);
-        rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K3l, K3t, dummyl, dummyt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-        K3dl = fma(ih, K1dl - K2dl, Ql) + Gl;
-        K3dt = fma(ih, K1dt - K2dt, Qt) + Gt;
+        // stage 3: F at Y3 = N + 2 K1 along Ydot3 = Ndot + 2 Kdot1
+        const double Y3el = Ndl + 2.0 * K1dl, Y3et = Ndt + 2.0 * K1dt;
+        rhs_eps(Nl + 2.0 * K1l, Nt + 2.0 * K1t, Y3el, Y3et, Ql, Qt, net, nd, ndd, ts, spare, rk, rkd, lane);
+        K3dl = fma(ih, K1dl - K2dl, Ql) + Gl[2];
+        K3dt = fma(ih, K1dt - K2dt, Qt) + Gt[2];
         if (ad) {
           K3dl += sg * K3l - hq * (K1l - kp.K2l);
           K3dt += sg * K3t - hq * (K1t - kp.K2t);
         }
         w_solve(K3dl, K3dt, c, a21, kp, dtr, ws, lane);
-        // stage 4: F at Y4 = N + 2 K1 + K3 along Ndot + 2 Kdot1 + Kdot3; Jdot K4 at N
-        rhs_tangent<false>(Nl + 2.0 * K1l + K3l, Nt + 2.0 * K1t + K3t, Y3el + K3dl, Y3et + K3dt, 0.0, 0.0, Ql, Qt,
-                           dummyl, dummyt, net, nd, ndd, ts, rk, rkd, lane);
-        rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K4l, K4t, dummyl, dummyt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-        K4dl = fma(ih, fma(-RODAS_C43, K3dl, K1dl - K2dl), Ql) + Gl;
-        K4dt = fma(ih, fma(-RODAS_C43, K3dt, K1dt - K2dt), Qt) + Gt;
+        // stage 4: F at Y4 = N + 2 K1 + K3 along Ndot + 2 Kdot1 + Kdot3
+        rhs_eps(Nl + 2.0 * K1l + K3l, Nt + 2.0 * K1t + K3t, Y3el + K3dl, Y3et + K3dt, Ql, Qt, net, nd, ndd, ts, spare, rk,
+                rkd, lane);
+        K4dl = fma(ih, fma(-RODAS_C43, K3dl, K1dl - K2dl), Ql) + Gl[3];
+        K4dt = fma(ih, fma(-RODAS_C43, K3dt, K1dt - K2dt), Qt) + Gt[3];
         if (ad) {
           K4dl += sg * K4l - hq * fma(-RODAS_C43, K3l, K1l - kp.K2l);
           K4dt += sg * K4t - hq * fma(-RODAS_C43, K3t, K1t - kp.K2t);
@@ -818,41 +900,43 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
         double end = 0.0;  // the error's tangent (adaptive contract)
         if (ok || ad) {
           // the try's tangent on its dense factors, as the tangent kernel's on the sparse ones
-          double Fel, Fet, Gl, Gt, Ql, Qt, dl, dtt;
+          double Fel, Fet, Ql, Qt, Gl[4], Gt[4];  // Fdot(N), Fdot(Y); Jdot K_i (eps-del parts)
           double K1dl, K1dt, K2dl, K2dt, K3dl, K3dt, K4dl, K4dt;
+          const double Kl[4] = {K1l, K2l, K3l, K4l}, Kt[4] = {K1t, K2t, K3t, K4t};
+          double* spare = ws + L_DV;
+          stage_products(Nl, Nt, Ndl, Ndt, Kl, Kt, Fel, Fet, Gl, Gt, net, nd, ndd, ts, spare, rk, rkd, lane);
+          K1dl = Fel + Gl[0];
+          K1dt = Fet + Gt[0];
+          // adaptive: W = I / (gamma h) - J moves with h, W Kdot = bdot + Jdot K + hdot / (gamma h^2) K, and the stages'
+          // K / h terms give -hdot / h^2 K
           const double sg = had * ih * ih / GAMMA, hq = had * ih * ih;
-          rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K1l, K1t, Fel, Fet, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-          K1dl = Fel + Gl;
-          K1dt = Fet + Gt;
           if (ad) {
             K1dl = fma(sg, K1l, K1dl);
             K1dt = fma(sg, K1t, K1dt);
           }
           dense_solve_pair(W, pr, dinv, yv, K1dl, K1dt, lane);
-          rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K2l, K2t, Ql, Qt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-          K2dl = fma(RODAS_C21 * ih, K1dl, Fel) + Gl;
-          K2dt = fma(RODAS_C21 * ih, K1dt, Fet) + Gt;
+          K2dl = fma(RODAS_C21 * ih, K1dl, Fel) + Gl[1];
+          K2dt = fma(RODAS_C21 * ih, K1dt, Fet) + Gt[1];
           if (ad) {
             K2dl += sg * K2l - hq * RODAS_C21 * K1l;
             K2dt += sg * K2t - hq * RODAS_C21 * K1t;
           }
           dense_solve_pair(W, pr, dinv, yv, K2dl, K2dt, lane);
+          // stage 3: F at Y3 = N + 2 K1 along Ydot3 = Ndot + 2 Kdot1
           const double Y3el = Ndl + 2.0 * K1dl, Y3et = Ndt + 2.0 * K1dt;
-          rhs_tangent<false>(Nl + 2.0 * K1l, Nt + 2.0 * K1t, Y3el, Y3et, 0.0, 0.0, Ql, Qt, dl, dtt, net, nd, ndd, ts,
-                             rk, rkd, lane);
-          rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K3l, K3t, dl, dtt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-          K3dl = fma(ih, K1dl - K2dl, Ql) + Gl;
-          K3dt = fma(ih, K1dt - K2dt, Qt) + Gt;
+          rhs_eps(Nl + 2.0 * K1l, Nt + 2.0 * K1t, Y3el, Y3et, Ql, Qt, net, nd, ndd, ts, spare, rk, rkd, lane);
+          K3dl = fma(ih, K1dl - K2dl, Ql) + Gl[2];
+          K3dt = fma(ih, K1dt - K2dt, Qt) + Gt[2];
           if (ad) {
             K3dl += sg * K3l - hq * (K1l - K2l);
             K3dt += sg * K3t - hq * (K1t - K2t);
           }
           dense_solve_pair(W, pr, dinv, yv, K3dl, K3dt, lane);
-          rhs_tangent<false>(Nl + 2.0 * K1l + K3l, Nt + 2.0 * K1t + K3t, Y3el + K3dl, Y3et + K3dt, 0.0, 0.0, Ql, Qt,
-                             dl, dtt, net, nd, ndd, ts, rk, rkd, lane);
-          rhs_tangent<true>(Nl, Nt, Ndl, Ndt, K4l, K4t, dl, dtt, Gl, Gt, net, nd, ndd, ts, rk, rkd, lane);
-          K4dl = fma(ih, fma(-RODAS_C43, K3dl, K1dl - K2dl), Ql) + Gl;
-          K4dt = fma(ih, fma(-RODAS_C43, K3dt, K1dt - K2dt), Qt) + Gt;
+          // stage 4: F at Y4 = N + 2 K1 + K3 along Ndot + 2 Kdot1 + Kdot3
+          rhs_eps(Nl + 2.0 * K1l + K3l, Nt + 2.0 * K1t + K3t, Y3el + K3dl, Y3et + K3dt, Ql, Qt, net, nd, ndd, ts, spare, rk,
+                  rkd, lane);
+          K4dl = fma(ih, fma(-RODAS_C43, K3dl, K1dl - K2dl), Ql) + Gl[3];
+          K4dt = fma(ih, fma(-RODAS_C43, K3dt, K1dt - K2dt), Qt) + Gt[3];
           if (ad) {
             K4dl += sg * K4l - hq * fma(-RODAS_C43, K3l, K1l - K2l);
             K4dt += sg * K4t - hq * fma(-RODAS_C43, K3t, K1t - K2t);
