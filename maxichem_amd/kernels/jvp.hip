@@ -784,7 +784,8 @@ __device__ __forceinline__ void dense_solve_pair(const double* W, const int* pr,
 // (W Kdot = bdot + Jdot K, plus the step's terms under the adaptive contract) on its threshold-pivoted factors. A
 // pass's first step min(h, dt split^k) takes the tangent of its smaller side (half of each at a tie), then that of
 // max(., H_MIN). The result's tangent goes through the guard's, as the tangent kernel's; a cell that still fails the
-// guard (flag 2) gets NaN. Workgroups of REC_WAVES wavefronts share each dense LU as mxc_recover's.
+// guard (flag 2) gets NaN. Workgroups of REC_WAVES wavefronts share each dense LU as mxc_recover's. One launch takes
+// every direction's pairs (direction, listed cell) from one queue, as mxc_jvp.
 extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
     mxc_jvp_recover(NetP __restrict__ net, const double* __restrict__ x0, const double* __restrict__ Ta,
                     const double* __restrict__ Pa, const double* __restrict__ dta, const double* __restrict__ hin,
@@ -795,9 +796,9 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
                     const double* __restrict__ Td, const double* __restrict__ Pd, const double* __restrict__ Jd,
                     double* __restrict__ xd, int adapt, const double* __restrict__ dtd, const double* __restrict__ hd,
                     double* __restrict__ hdo, const double* __restrict__ lmd, const double* __restrict__ rcd,
-                    double* __restrict__ rsc) {
-  const int nfl = count[COUNT_RECOMPUTED];
-  if ((int)blockIdx.x >= nfl) return;
+                    int B, int D, double* __restrict__ rsc) {
+  const int nfl = count[COUNT_RECOMPUTED], pairs = nfl * D;
+  if ((int)blockIdx.x >= pairs) return;
   extern __shared__ double lds[];
   const int lane = (int)(threadIdx.x & (WAVE - 1)), wv = (int)(threadIdx.x / WAVE);
   double* ws = lds;
@@ -825,22 +826,23 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   LeadRow a21;
   const bool ad = adapt != 0;
   int q = (int)blockIdx.x;
-  while (q < nfl) {
-    const int cell = list[q];
+  while (q < pairs) {
+    const int dir = q / nfl, cell = list[q - dir * nfl];
+    const size_t dc = (size_t)dir * B + cell;  // the pair's row in the per-direction arrays
     const double Tc = Ta[cell], dt = dta[cell], nd = Pa[cell] / (KBOLTZ * Tc);
     const double* xr = x0 + (size_t)cell * NS;
-    const double* xdr = x0d + (size_t)cell * NS;
+    const double* xdr = x0d + dc * NS;
     const double* Jc = NJ ? Jin + (size_t)cell * NJ : nullptr;
     const double* lmc = lm ? lm + (size_t)cell * NR : nullptr;
     cell_rates(ws, rk, Tc, nd, net, Jc, lane, lmc);
-    const double Tdc = Td ? Td[cell] : 0.0, Pdc = Pd ? Pd[cell] : 0.0;
+    const double Tdc = Td ? Td[dc] : 0.0, Pdc = Pd ? Pd[dc] : 0.0;
     const double ndd = nd * (Pdc / Pa[cell] - Tdc / Tc);
-    rates_tangent(ts, rkd, Tc, Tdc, nd, ndd, net, Jc, (NJ && Jd) ? Jd + (size_t)cell * NJ : nullptr, lmc,
-                  lmd ? lmd + (size_t)cell * NR : nullptr, rcd, lane);
+    rates_tangent(ts, rkd, Tc, Tdc, nd, ndd, net, Jc, (NJ && Jd) ? Jd + dc * NJ : nullptr, lmc,
+                  lmd ? lmd + dc * NR : nullptr, rcd ? rcd + (size_t)dir * NR * 9 : nullptr, lane);
     const double h0 = isfinite(hin[cell]) ? hin[cell] : dt;
     const double m = fmin(h0, dt);
-    const double dtdc = (ad && dtd) ? dtd[cell] : 0.0;
-    const double h0d = !ad ? 0.0 : (isfinite(hin[cell]) ? (hd ? hd[cell] : 0.0) : dtdc);
+    const double dtdc = (ad && dtd) ? dtd[dc] : 0.0;
+    const double h0d = !ad ? 0.0 : (isfinite(hin[cell]) ? (hd ? hd[dc] : 0.0) : dtdc);
     const double md = h0 < dt ? h0d : (h0 > dt ? dtdc : 0.5 * (h0d + dtdc));  // m's tangent
     int ntry = 0;
     for (int pass = 0;; pass++) {
@@ -975,7 +977,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
       const int code = __builtin_amdgcn_readfirstlane(
           guard_wave(Nl, Nt, xr, xout + (size_t)cell * NS, dn != 0, s.nok, atol, net, lane));
       if (code == GUARD_DRIFT && pass < REC_RETRIES) continue;  // only drifted: again, with a smaller first try
-      double* xdo = xd + (size_t)cell * NS;
+      double* xdo = xd + dc * NS;
       if (code == 0) {
         guard_tangent(Nl, Nt, Ndl, Ndt, xr, xdr, xdo, net, lane);
       } else {
@@ -984,12 +986,14 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
       int nx = 0;
       if (lane == 0) {
         hio[cell] = s.h;
-        if (hdo) hdo[cell] = !ad ? 0.0 : (code == 0 ? hdot : DNAN);
+        if (hdo) hdo[dc] = !ad ? 0.0 : (code == 0 ? hdot : DNAN);
         doneo[cell] = code ? 0 : dn;  // done: finished and passing the guard
         noko[cell] = s.nok;
         redo[cell] = code ? 2 : 1;
-        if (tries) tries[cell] += (double)ntry;
-        atomicAdd(count + (code ? COUNT_STILL_FAILED : COUNT_RECOVERED), 1);
+        if (dir == 0) {  // direction 0's pair keeps the counts and the tries; the others write the same results
+          if (tries) tries[cell] += (double)ntry;
+          atomicAdd(count + (code ? COUNT_STILL_FAILED : COUNT_RECOVERED), 1);
+        }
         nx = (int)gridDim.x + atomicAdd(count + COUNT_RECOVERY_QUEUE, 1);
       }
       q = __builtin_amdgcn_readfirstlane(nx);

@@ -219,33 +219,27 @@ class ADSolver(CudaSolver):
                 p(dh), p(hd), p(lm), p(dlm), p(drc), ctypes.c_int(D), p(self._jrsc)]  # fmt: skip
         if B:
             _hip.launch(self._jvp, max(1, min(B * D, self.max_blocks_jvp)), WAVE, self.lds_jvp, stream, args)
-        # the cells the guard failed: the recovery's result with each direction's tangent. Direction 0's launch keeps
-        # the counts and the tries; the others run on a copy of the counts as the tangent kernel left them (the list's
-        # length), write the same results again and leave the tries alone
-        listed = self.count.clone()
-
-        def row(a, d):
-            return None if a is None else a[d]
-
-        for d in range(D):
-            count = self.count if d == 0 else listed.clone()
-            rec_args = [p(net), p(x), p(T), p(P), p(dt), p(h), p(xo), p(ho), p(done), p(nok), p(redo), p(lst), p(count),
-                        p(self.tries if d == 0 else None), p(jx), ctypes.c_double(rtol), ctypes.c_double(atol),
-                        ctypes.c_int(REC_STEPS * max_steps), p(lm), p(dx[d]), p(row(dT, d)), p(row(dP, d)),
-                        p(row(dJ, d)), p(xd[d]), ctypes.c_int(int(bool(adapt))), p(row(ddt, d)), p(row(dh, d)),
-                        p(hd[d]), p(row(dlm, d)), p(row(drc, d)), p(self._jrsc)]  # fmt: skip
-            _hip.launch(self._jvp_recover, max(1, min(B, self.rec_blocks_jvp)), WAVE * _kernels.REC_WAVES,
-                        self.lds_jvp_rec, stream, rec_args)  # fmt: skip
+        # the cells the guard failed: the recovery's result with every direction's tangent, in one launch (direction 0's
+        # pairs keep the counts and the tries)
+        rec_args = [p(net), p(x), p(T), p(P), p(dt), p(h), p(xo), p(ho), p(done), p(nok), p(redo), p(lst), p(self.count),
+                    p(self.tries), p(jx), ctypes.c_double(rtol), ctypes.c_double(atol),
+                    ctypes.c_int(REC_STEPS * max_steps), p(lm), p(dx), p(dT), p(dP), p(dJ), p(xd),
+                    ctypes.c_int(int(bool(adapt))), p(ddt), p(dh), p(hd), p(dlm), p(drc), ctypes.c_int(B),
+                    ctypes.c_int(D), p(self._jrsc)]  # fmt: skip
+        _hip.launch(self._jvp_recover, max(1, min(B * D, self.rec_blocks_jvp)), WAVE * _kernels.REC_WAVES,
+                    self.lds_jvp_rec, stream, rec_args)  # fmt: skip
         self._status = status
         return xo, ho, done, nok, redo
 
-    def _column_chunks(self, columns, B: int):
-        """The vjp's columns in launches of at most DMAX directions, each launch's unit tangents within
-        COLUMN_BYTES."""
+    def _column_chunks(self, columns: int, B: int):
+        """The vjp's columns [first, last) of each launch: as many directions as their unit tangents and outputs take
+        COLUMN_BYTES. A launch lasts at least its costliest cell's tries and a host visit costs about 0.1 ms, so fewer,
+        fuller launches (64 NCHO cells, 509 columns: 41 ms in eight launches with a recovery launch per column, 13.5 ms
+        in one)."""
         per = 8 * B * (2 * self.ns + 4 + self.nj + self.nr)  # one direction's tangents and outputs, at most
-        size = max(1, min(DMAX, COLUMN_BYTES // max(per, 1)))
-        for i in range(0, len(columns), size):
-            yield columns[i : i + size]
+        size = max(1, min(COLUMN_BYTES // max(per, 1), columns))
+        for i in range(0, columns, size):
+            yield i, min(columns, i + size)
 
     def vjp(self, x, T, P, dt, h, gx, *, gh=None, lm=None, rc=None, adapt: bool = True, rtol: float = DEFAULT_RTOL,
             atol: float = ATOL, max_steps: int = DEFAULT_MAX_STEPS, J=None, rates: bool = True) -> VjpResult:  # fmt: skip
@@ -255,14 +249,14 @@ class ADSolver(CudaSolver):
 
         Built from the tangent by columns, not by a reverse pass: one tangent direction per input coordinate (each
         of x's S entries, T, P, each photolysis branch, under adapt=True dt and h, and with rates each thermal
-        reaction's multiplier), every cell along the same unit direction, up to 64 directions in one launch, and each
-        cell's cotangent gx . dx + gh dh of its column. A photolysis branch's multiplier cotangent is J times J's
-        (kf = J exp(lm)); the rate table's is reduced from the multipliers' by mxc_rc_cotangent (a multiplier and the
-        law enter a reaction's coefficients alike, the law's share 1 - wA of the collision limit). Its work is S + 2 +
-        branches (+ 2) tangent calls, and the thermal reactions' count more with rates (rates=False leaves the
-        cotangents of lm and rc None); a small batch runs its columns side by side. Under the
-        frozen contract the cotangents of dt and h are zero. A cell that still fails the guard (flag 2) has NaN
-        cotangents and is left out of the rate table's sum (fallback["still_failed"] counts them)."""
+        reaction's multiplier), every cell along the same unit direction, as many directions in one launch as
+        COLUMN_BYTES hold, and each cell's cotangent gx . dx + gh dh of its column. A photolysis branch's multiplier
+        cotangent is J times J's (kf = J exp(lm)); the rate table's is reduced from the multipliers' by
+        mxc_rc_cotangent (a multiplier and the law enter a reaction's coefficients alike, the law's share 1 - wA of the
+        collision limit). Its work is S + 2 + branches (+ 2) tangent calls, and the thermal reactions' count more with
+        rates (rates=False leaves the cotangents of lm and rc None); a small batch runs its columns side by side.
+        Under the frozen contract the cotangents of dt and h are zero. A cell that still fails the guard (flag 2) has
+        NaN cotangents and is left out of the rate table's sum (fallback["still_failed"] counts them)."""
         self.flag = None
         self._require_open()
         B = check_inputs(self.dev, self.ns, x, T, P, dt, h, rtol, atol, max_steps)
@@ -281,38 +275,45 @@ class ADSolver(CudaSolver):
                            rc=torch.empty(self.nr, ARRHENIUS_COLUMNS, dtype=torch.float64, device=self.dev)
                            if rates else None,
                            J=torch.empty(B, self.nj, dtype=torch.float64, device=self.dev) if self.nj else None)  # fmt: skip
-            # the input coordinates, each a unit direction for every cell at once: (what, index, where its
-            # cotangent goes)
-            columns = [("x", s, g.x[:, s]) for s in range(self.ns)] + [("T", 0, g.T), ("P", 0, g.P)]
-            columns += [("J", b, g.J[:, b]) for b in range(self.nj)]
+            # the input coordinates, each a unit direction for every cell at once: (what, where their cotangents go), in
+            # the columns' order
+            kinds = [("x", g.x), ("T", g.T[:, None]), ("P", g.P[:, None])]
+            kinds += [("J", g.J)] if self.nj else []
             if adapt:  # dt and h enter under the adaptive contract
-                columns += [("dt", 0, g.dt), ("h", 0, g.h)]
+                kinds += [("dt", g.dt[:, None]), ("h", g.h[:, None])]
             if rates:  # the thermal reactions' multipliers
-                columns += [("lm", r, g.lm[:, r]) for r in range(self.tab.nrt)]
+                kinds += [("lm", g.lm[:, : self.tab.nrt])]
+            columns = sum(dest.shape[1] for _, dest in kinds)
             result = None
-            for chunk in self._column_chunks(columns, B):
-                D = len(chunk)
-                kinds = {k for k, _, _ in chunk}
+            for c0, c1 in self._column_chunks(columns, B):
+                D = c1 - c0
                 f64 = {"dtype": torch.float64, "device": self.dev}
-                dx = torch.zeros(D, B, self.ns, **f64)
-                dT, dP, ddt, dh = (torch.zeros(D, B, **f64) if k in kinds else None for k in ("T", "P", "dt", "h"))
-                dJ = torch.zeros(D, B, self.nj, **f64) if "J" in kinds else None
-                dlm = torch.zeros(D, B, self.nr, **f64) if "lm" in kinds else None
-                unit = {"x": dx, "T": dT, "P": dP, "dt": ddt, "h": dh, "J": dJ, "lm": dlm}
-                for d, (k, i, _) in enumerate(chunk):
+                # each kind's columns in this launch: its directions [a, b), from its column lo
+                spans, at = [], 0
+                for k, dest in kinds:
+                    lo, hi = max(c0, at), min(c1, at + dest.shape[1])
+                    if lo < hi:
+                        spans.append((k, dest, lo - c0, hi - c0, lo - at))
+                    at += dest.shape[1]
+                unit = {"x": torch.zeros(D, B, self.ns, **f64)}
+                for k, _, a, b, lo in spans:
                     if k in ("x", "J", "lm"):
-                        unit[k][d, :, i] = 1.0
+                        if k not in unit:
+                            unit[k] = torch.zeros(D, B, {"J": self.nj, "lm": self.nr}[k], **f64)
+                        torch.diagonal(unit[k][a:b], lo, 0, 2)[:, : b - a].fill_(1.0)  # direction a + i: column lo + i
                     else:
-                        unit[k][d] = 1.0
+                        unit[k] = torch.zeros(D, B, **f64)
+                        unit[k][a:b] = 1.0
                 xd = torch.empty(D, B, self.ns, **f64)
                 hd = torch.empty(D, B, **f64)
-                result = self._jvp_launch(x, T, P, dt, h, jx, rtol, atol, max_steps, B, D, dx, dT, dP, dJ, xd, adapt,
-                                          ddt, dh, hd, lm, dlm, None, net)  # fmt: skip
-                out = torch.einsum("dbs,bs->db", xd, gx)
+                result = self._jvp_launch(x, T, P, dt, h, jx, rtol, atol, max_steps, B, D, unit["x"], unit.get("T"),
+                                          unit.get("P"), unit.get("J"), xd, adapt, unit.get("dt"), unit.get("h"), hd, lm,
+                                          unit.get("lm"), None, net)  # fmt: skip
+                out = torch.cat([torch.einsum("dbs,bs->db", q, gx) for q in xd.split(DMAX)])
                 if gh is not None and adapt:
                     out += hd * gh
-                for d, (_, _, dest) in enumerate(chunk):
-                    dest.copy_(out[d])
+                for _, dest, a, b, lo in spans:
+                    dest[:, lo : lo + b - a].copy_(out[a:b].T)
             if rates and self.nj:  # a branch's kf = J exp(lm): d/dlm = J d/dJ
                 g.lm[:, self.tab.nrt:] = jx * g.J
             xo, ho, done, nok, redo = result
