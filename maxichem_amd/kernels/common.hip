@@ -317,37 +317,56 @@ __device__ __forceinline__ void lds_add(double* p, double d) {
 // places in dst, which hold 0 before (padding words add 0 to a place of their lane's). The adds are LDS atomics: an
 // entry's terms come from one lane, so they are taken in order, and a word costs no running sum, no select and no
 // wait: 9 instructions, where a running sum with its selects took 19 (NCHO, cycles of one wavefront per try: the
-// Jacobian 23.0k -> 17.4k, the three right-hand sides 21.4k -> 17.9k). The words of STREAM_BATCH rounds are loaded together, ahead of their terms, so that their latency is paid once
-// per batch: whole batches in a loop, then the last rounds as a batch of their own (the rounds are known when the kernel
-// is built). SIGNED: the terms may be negative; else the word's sign bit is put in place of theirs.
-template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, bool SIGNED, typename WP>
-__device__ __forceinline__ void stream_sum(WP __restrict__ words, int rounds, const double* src, double* dst,
-                                           int lane) {
-  auto batch = [&](int q0, int n) {  // rounds q0 .. q0 + n - 1, n <= STREAM_BATCH
-    u32 w[STREAM_BATCH];
+// Jacobian 23.0k -> 17.4k, the three right-hand sides 21.4k -> 17.9k). The words go a batch of STREAM_BATCH rounds at a
+// time, each batch loaded before the terms of the one before it are read (the first by the caller, ahead of what makes
+// the terms), so that no batch waits for its words (NCHO, with the rates ahead in rhs: 256 cold cells 17.3 -> 16.6 ms,
+// 65,536 settled 7.5 -> 7.15 ms). SIGNED: the terms may be negative; else the word's sign bit is put in place of theirs.
+using StreamWords = u32[STREAM_BATCH];
+
+// Batch q0's words of a stream (rounds q0 .. , those past the stream's end left as they are).
+template <int ROUNDS, typename WP>
+__device__ __forceinline__ void load_words(WP words, int q0, StreamWords& w, int lane) {
+#pragma unroll
+  for (int i = 0; i < STREAM_BATCH; i++)
+    if (q0 + i < ROUNDS) w[i] = words[(q0 + i) * WAVE + lane];
+}
+
+// w: the first batch's words. next(w): called when the last batch's words are in use, to load another stream's.
+template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, bool SIGNED, int ROUNDS, typename WP, typename Next>
+__device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const double* src, double* dst, int lane, Next next) {
+  constexpr int LAST = ROUNDS > 0 ? (ROUNDS - 1) / STREAM_BATCH * STREAM_BATCH : 0;  // the last batch's first round
+  auto batch = [&](int n, auto load) {  // n <= STREAM_BATCH rounds
+    StreamWords cur;
     double d[STREAM_BATCH];
 #pragma unroll
-    for (int i = 0; i < STREAM_BATCH; i++)
-      if (i < n) w[i] = words[(q0 + i) * WAVE + lane];
+    for (int i = 0; i < STREAM_BATCH; i++) cur[i] = i < n ? w[i] : 0;
+    load();
 #pragma unroll
     for (int i = 0; i < STREAM_BATCH; i++)
-      if (i < n) d[i] = src[w[i] & IDX_MASK];
+      if (i < n) d[i] = src[cur[i] & IDX_MASK];
 #pragma unroll
     for (int i = 0; i < STREAM_BATCH; i++) {
       if (i >= n) break;
-      lds_add(dst + ((w[i] >> DEST) & DEST_MASK), term<DBL, SIGNED>(w[i], d[i]));
+      lds_add(dst + ((cur[i] >> DEST) & DEST_MASK), term<DBL, SIGNED>(cur[i], d[i]));
     }
   };
-  const int full = rounds / STREAM_BATCH * STREAM_BATCH;
 #pragma unroll 1
-  for (int q0 = 0; q0 < full; q0 += STREAM_BATCH) batch(q0, STREAM_BATCH);
-  if (rounds > full) batch(full, rounds - full);
+  for (int q0 = 0; q0 < LAST; q0 += STREAM_BATCH)
+    batch(STREAM_BATCH, [&] {
+#pragma unroll
+      for (int i = 0; i < STREAM_BATCH; i++) {  // past the end: the last round's words, which are not used
+        const int q = q0 + STREAM_BATCH + i;
+        w[i] = words[(q < ROUNDS ? q : ROUNDS - 1) * WAVE + lane];
+      }
+    });
+  batch(ROUNDS - LAST, [&] { next(w); });
 }
 
 // One Jacobian stream into the cell's LDS: entries of -Jn at their offsets.
-template <typename WP>
-__device__ __forceinline__ void jac_stream(WP __restrict__ words, int rounds, const double* DV, double* ws, int lane) {
-  stream_sum<T_IDX_MASK, T_DBL, T_DEST, T_DEST_MASK, false>(words, rounds, DV, ws, lane);  // dv terms are not negative
+template <int ROUNDS, typename WP, typename Next>
+__device__ __forceinline__ void jac_stream(WP words, StreamWords& w, const double* DV, double* ws, int lane, Next next) {
+  // dv terms are not negative
+  stream_sum<T_IDX_MASK, T_DBL, T_DEST, T_DEST_MASK, false, ROUNDS>(words, w, DV, ws, lane, next);
 }
 
 // The stream words in the workgroup's LDS (WORDS_LDS: the call kernel copies them there at its start, after its
@@ -387,13 +406,24 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
   // spare lanes read reaction NR - 1), so none waits on the branch that ends a lane's rounds
   u64 wr[RROUNDS];
   int fr[JAC ? RROUNDS : 1];
+  double fq[RROUNDS], bq[RROUNDS];
+  StreamWords sw;
+  auto svp = [&] {
+    if constexpr (LW)
+      return lds_words(ws) + W_SV;
+    else
+      return svw;
+  }();
   const u32 rpl = rowp[lane < K0 ? lane : 0], rpt = rowp[K0 + (lane < NT ? lane : 0)];  // each row's S v pieces
 #pragma unroll
   for (int q = 0; q < RROUNDS; q++) {
     const int r = q * WAVE + lane < NR ? q * WAVE + lane : NR - 1;
     wr[q] = rxe[r];
     if (JAC) fr[q] = rf[r];
+    fq[q] = kf[r];
+    bq[q] = kr[r];
   }
+  load_words<SV_ROUNDS>(svp, 0, sw, lane);
 #pragma unroll
   for (int q = 0; q < RROUNDS; q++) {
     const int r = q * WAVE + lane;
@@ -401,7 +431,7 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
     const u64 w = wr[q];
     const double n0 = n[species_of(w, 0)], n1 = n[species_of(w, 1)], n2 = n[species_of(w, 2)];
     const double n3 = n[species_of(w, 3)], n4 = n[species_of(w, 4)], n5 = n[species_of(w, 5)];
-    const double f = kf[r], b = kr[r];
+    const double f = fq[q], b = bq[q];
     V[r] = f * n0 * n1 * n2 - b * n3 * n4 * n5;
     if (JAC) {
       const int fl = fr[JAC ? q : 0];
@@ -426,10 +456,7 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
     if (i + lane < NPART) part[i + lane] = 0.0;
   if (lane == 0) V[NR] = 0.0;  // the S v stream's padding term
   wave_sync();
-  if constexpr (LW)
-    stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true>(lds_words(ws) + W_SV, SV_ROUNDS, V, part, lane);
-  else
-    stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true>(svw, SV_ROUNDS, V, part, lane);
+  stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true, SV_ROUNDS>(svp, sw, V, part, lane, [](StreamWords&) {});
   wave_sync();
   // each row's pieces in order; the reads go out together (a row of fewer pieces than the most reads within part)
   auto row = [&](u32 rp) {
@@ -462,12 +489,21 @@ struct IntSeq : Seq<K...> {};
 template <int N>
 using Steps = __make_integer_seq<IntSeq, int, N>;
 
+template <bool LW, int CH>
+__device__ __forceinline__ auto chunk_words(NetP net, const double* ws) {
+  if constexpr (LW)
+    return lds_words(ws) + W_CH + CH_OFF[CH] * WAVE;
+  else
+    return opaque(net)->chw + CH_OFF[CH] * WAVE;
+}
+
 // One chunk of CHUNK columns of the trailing rows' -Jn, through the staging area (column-major) into sink.chunk, and
 // its part of -Jn N. Chunks 0 .. NLCH - 1 hold the lead columns (K0 > 0 means NT == WAVE: every lane has a trailing
 // row), the others the trailing columns. cd: the row's own diagonal entry, which the chunk streams do not hold.
+// w: the chunk's first words, then the next chunk's.
 template <bool LW, int CH, typename Sink>
-__device__ __forceinline__ void jac_chunk(Sink& sink, double cd, double Nl, double Nt, double& mt, const double* xv,
-                                          NetP net, double* ws, int lane) {
+__device__ __forceinline__ void jac_chunk(Sink& sink, StreamWords& w, double cd, double Nl, double Nt, double& mt,
+                                          const double* xv, NetP net, double* ws, int lane) {
   const double* DV = ws + L_DV;
   double* stage = ws + L_STAGE;
   constexpr int C0 = (CH < NLCH ? CH : CH - NLCH) * CHUNK, NC = CH < NLCH ? K0 : NT;  // its first column, of NC
@@ -477,10 +513,9 @@ __device__ __forceinline__ void jac_chunk(Sink& sink, double cd, double Nl, doub
     if (CH >= NLCH && lane / CHUNK == CH - NLCH) stage[(lane % CHUNK) * NT + lane] = cd;
   }
   wave_sync();
-  if constexpr (LW)
-    jac_stream(lds_words(ws) + W_CH + CH_OFF[CH] * WAVE, CH_ROUNDS[CH], DV, ws, lane);
-  else
-    jac_stream(opaque(net)->chw + CH_OFF[CH] * WAVE, CH_ROUNDS[CH], DV, ws, lane);
+  jac_stream<CH_ROUNDS[CH]>(chunk_words<LW, CH>(net, ws), w, DV, ws, lane, [&](StreamWords& v) {
+    if constexpr (CH + 1 < NCH) load_words<CH_ROUNDS[CH + 1]>(chunk_words<LW, CH + 1>(net, ws), 0, v, lane);
+  });
   wave_sync();
   // N_j for -Jn N as wave-uniform values: with few lead rows from the exchange vector (same-address LDS reads, kept in
   // their chunk: hoisted ahead, they would hold a register pair each), else by v_readlane
@@ -500,9 +535,9 @@ __device__ __forceinline__ void jac_chunk(Sink& sink, double cd, double Nl, doub
 }
 
 template <bool LW, typename Sink, int... CH>
-__device__ __forceinline__ void jac_chunks(Seq<CH...>, Sink& sink, double cd, double Nl, double Nt, double& mt,
+__device__ __forceinline__ void jac_chunks(Seq<CH...>, Sink& sink, StreamWords& w, double cd, double Nl, double Nt, double& mt,
                                            const double* xv, NetP net, double* ws, int lane) {
-  (jac_chunk<LW, CH>(sink, cd, Nl, Nt, mt, xv, net, ws, lane), ...);
+  (jac_chunk<LW, CH>(sink, w, cd, Nl, Nt, mt, xv, net, ws, lane), ...);
 }
 
 // -Jn: the lead rows into LEAD (LDS), the trailing rows to sink, from the dv terms in DV; then u = w = S v / nd -
@@ -513,6 +548,20 @@ __device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, d
   lane = opaque_lane(lane);
   ws = opaque_lds(ws);
   double* DV = ws + L_DV;
+  auto dwords = [&] {
+    if constexpr (LW)
+      return lds_words(ws) + W_DIAG;
+    else
+      return opaque(net)->diagw;
+  }();
+  auto lwords = [&] {
+    if constexpr (LW)
+      return lds_words(ws) + W_LEAD;
+    else
+      return opaque(net)->leadw;
+  }();
+  StreamWords w;
+  load_words<DIAG_ROUNDS>(dwords, 0, w, lane);
   for (int s = lane; s < L_NVEC; s += WAVE) ws[s] = 0.0;  // LEAD
   if (lane < NT) ws[L_DIAG + lane] = 0.0;                   // a species in no reaction has no diagonal term
   if (lane == 0) DV[NDV] = 0.0;                             // the padding words' term
@@ -521,13 +570,10 @@ __device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, d
   if (lane < K0) xv[lane] = Nl;
   if (lane < NT) xv[K0 + lane] = Nt;
   wave_sync();
-  if constexpr (LW) {
-    jac_stream(lds_words(ws) + W_DIAG, DIAG_ROUNDS, DV, ws, lane);
-    jac_stream(lds_words(ws) + W_LEAD, LEAD_ROUNDS, DV, ws, lane);
-  } else {
-    jac_stream(opaque(net)->diagw, DIAG_ROUNDS, DV, ws, lane);
-    jac_stream(opaque(net)->leadw, LEAD_ROUNDS, DV, ws, lane);
-  }
+  jac_stream<DIAG_ROUNDS>(dwords, w, DV, ws, lane, [&](StreamWords& v) { load_words<LEAD_ROUNDS>(lwords, 0, v, lane); });
+  jac_stream<LEAD_ROUNDS>(lwords, w, DV, ws, lane, [&](StreamWords& v) {
+    load_words<CH_ROUNDS[0]>(chunk_words<LW, 0>(net, ws), 0, v, lane);
+  });
   wave_sync();
   // -Jn N in FP64: the lead rows through the exchange vector, then the trailing rows chunk by chunk (their lead
   // columns, then the trailing ones)
@@ -556,7 +602,7 @@ __device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, d
     }
   }
   const double cd = lane < NT ? ws[L_DIAG + lane] : 0.0;
-  jac_chunks<LW>(Steps<NCH>{}, sink, cd, Nl, Nt, mt, xv, net, ws, lane);
+  jac_chunks<LW>(Steps<NCH>{}, sink, w, cd, Nl, Nt, mt, xv, net, ws, lane);
   ul = u0l + ml / ntot;
   ut = lane < NT ? u0t + mt / ntot : 0.0;
   wave_sync();
