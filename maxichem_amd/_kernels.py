@@ -86,7 +86,7 @@ SIMDS = 4  # SIMDs per compute unit
 
 def words_in_lds(tab: Tables, cpw: int, mixed: bool = False, wps: int = 1, rates_global: bool = False) -> bool:
     """Whether the call kernel keeps the stream words in its workgroup's LDS (read with the LDS's latency instead of
-    the caches'; measured 2.6 % faster on NCHO): the plain form only, when the words fit beside the workgroup's cells
+    the caches'): the plain form only, when the words fit beside the workgroup's cells
     without lowering the cells a compute unit holds."""
     if mixed:
         return False

@@ -318,28 +318,36 @@ __device__ __forceinline__ void lds_add(double* p, double d) {
 // entry's terms come from one lane, so they are taken in order, and a word costs no running sum, no select and no
 // wait: 9 instructions, where a running sum with its selects took 19 (NCHO, cycles of one wavefront per try: the
 // Jacobian 23.0k -> 17.4k, the three right-hand sides 21.4k -> 17.9k). The words go a batch of STREAM_BATCH rounds at a
-// time, each batch loaded before the terms of the one before it are read (the first by the caller, ahead of what makes
-// the terms), so that no batch waits for its words (NCHO, with the rates ahead in rhs: 256 cold cells 17.3 -> 16.6 ms,
-// 65,536 settled 7.5 -> 7.15 ms). SIGNED: the terms may be negative; else the word's sign bit is put in place of theirs.
+// time: whole batches in a loop, then the last rounds as a batch of their own (the rounds are known when the kernel is
+// built). The last batch's words are loaded before the terms of the batch ahead of it are read, those of a stream of one
+// batch by its caller, so that it does not wait for them (NCHO, with the rates ahead in rhs: 256 cold cells
+// 17.3 -> 16.6 ms, 65,536 settled 7.5 -> 7.15 ms; the loop's words carried from batch to batch as well: no faster, and
+// the module takes 62 s to compile instead of 40). SIGNED: the terms may be negative; else the word's sign bit is put in
+// place of theirs.
 using StreamWords = u32[STREAM_BATCH];
 
-// Batch q0's words of a stream (rounds q0 .. , those past the stream's end left as they are).
+// The words of a stream's rounds from q0 on, at most a batch of them.
 template <int ROUNDS, typename WP>
 __device__ __forceinline__ void load_words(WP words, int q0, StreamWords& w, int lane) {
 #pragma unroll
   for (int i = 0; i < STREAM_BATCH; i++)
     if (q0 + i < ROUNDS) w[i] = words[(q0 + i) * WAVE + lane];
 }
+// What a stream's caller loads ahead: the words of a stream of one batch.
+template <int ROUNDS, typename WP>
+__device__ __forceinline__ void load_ahead(WP words, StreamWords& w, int lane) {
+  if constexpr (ROUNDS <= STREAM_BATCH) load_words<ROUNDS>(words, 0, w, lane);
+}
 
-// w: the first batch's words. next(w): called when the last batch's words are in use, to load another stream's.
+// w: what load_ahead loaded. next(w): called when the last batch's words are in use, to load another stream's ahead.
 template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, bool SIGNED, int ROUNDS, typename WP, typename Next>
 __device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const double* src, double* dst, int lane, Next next) {
   constexpr int LAST = ROUNDS > 0 ? (ROUNDS - 1) / STREAM_BATCH * STREAM_BATCH : 0;  // the last batch's first round
-  auto batch = [&](int n, auto load) {  // n <= STREAM_BATCH rounds
+  auto batch = [&](StreamWords& from, int n, auto load) {  // n <= STREAM_BATCH rounds
     StreamWords cur;
     double d[STREAM_BATCH];
 #pragma unroll
-    for (int i = 0; i < STREAM_BATCH; i++) cur[i] = i < n ? w[i] : 0;
+    for (int i = 0; i < STREAM_BATCH; i++) cur[i] = i < n ? from[i] : 0;
     load();
 #pragma unroll
     for (int i = 0; i < STREAM_BATCH; i++)
@@ -351,15 +359,15 @@ __device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const doubl
     }
   };
 #pragma unroll 1
-  for (int q0 = 0; q0 < LAST; q0 += STREAM_BATCH)
-    batch(STREAM_BATCH, [&] {
+  for (int q0 = 0; q0 < LAST; q0 += STREAM_BATCH) {
+    StreamWords v;
 #pragma unroll
-      for (int i = 0; i < STREAM_BATCH; i++) {  // past the end: the last round's words, which are not used
-        const int q = q0 + STREAM_BATCH + i;
-        w[i] = words[(q < ROUNDS ? q : ROUNDS - 1) * WAVE + lane];
-      }
+    for (int i = 0; i < STREAM_BATCH; i++) v[i] = words[(q0 + i) * WAVE + lane];
+    batch(v, STREAM_BATCH, [&] {
+      if (q0 + STREAM_BATCH >= LAST) load_words<ROUNDS>(words, LAST, w, lane);
     });
-  batch(ROUNDS - LAST, [&] { next(w); });
+  }
+  batch(w, ROUNDS - LAST, [&] { next(w); });
 }
 
 // One Jacobian stream into the cell's LDS: entries of -Jn at their offsets.
@@ -423,7 +431,7 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
     fq[q] = kf[r];
     bq[q] = kr[r];
   }
-  load_words<SV_ROUNDS>(svp, 0, sw, lane);
+  load_ahead<SV_ROUNDS>(svp, sw, lane);
 #pragma unroll
   for (int q = 0; q < RROUNDS; q++) {
     const int r = q * WAVE + lane;
@@ -514,7 +522,7 @@ __device__ __forceinline__ void jac_chunk(Sink& sink, StreamWords& w, double cd,
   }
   wave_sync();
   jac_stream<CH_ROUNDS[CH]>(chunk_words<LW, CH>(net, ws), w, DV, ws, lane, [&](StreamWords& v) {
-    if constexpr (CH + 1 < NCH) load_words<CH_ROUNDS[CH + 1]>(chunk_words<LW, CH + 1>(net, ws), 0, v, lane);
+    if constexpr (CH + 1 < NCH) load_ahead<CH_ROUNDS[CH + 1]>(chunk_words<LW, CH + 1>(net, ws), v, lane);
   });
   wave_sync();
   // N_j for -Jn N as wave-uniform values: with few lead rows from the exchange vector (same-address LDS reads, kept in
@@ -561,7 +569,7 @@ __device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, d
       return opaque(net)->leadw;
   }();
   StreamWords w;
-  load_words<DIAG_ROUNDS>(dwords, 0, w, lane);
+  load_ahead<DIAG_ROUNDS>(dwords, w, lane);
   for (int s = lane; s < L_NVEC; s += WAVE) ws[s] = 0.0;  // LEAD
   if (lane < NT) ws[L_DIAG + lane] = 0.0;                   // a species in no reaction has no diagonal term
   if (lane == 0) DV[NDV] = 0.0;                             // the padding words' term
@@ -570,9 +578,9 @@ __device__ __forceinline__ void jac_assemble(Sink& sink, double Nl, double Nt, d
   if (lane < K0) xv[lane] = Nl;
   if (lane < NT) xv[K0 + lane] = Nt;
   wave_sync();
-  jac_stream<DIAG_ROUNDS>(dwords, w, DV, ws, lane, [&](StreamWords& v) { load_words<LEAD_ROUNDS>(lwords, 0, v, lane); });
+  jac_stream<DIAG_ROUNDS>(dwords, w, DV, ws, lane, [&](StreamWords& v) { load_ahead<LEAD_ROUNDS>(lwords, v, lane); });
   jac_stream<LEAD_ROUNDS>(lwords, w, DV, ws, lane, [&](StreamWords& v) {
-    load_words<CH_ROUNDS[0]>(chunk_words<LW, 0>(net, ws), 0, v, lane);
+    load_ahead<CH_ROUNDS[0]>(chunk_words<LW, 0>(net, ws), v, lane);
   });
   wave_sync();
   // -Jn N in FP64: the lead rows through the exchange vector, then the trailing rows chunk by chunk (their lead

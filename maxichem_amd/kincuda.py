@@ -68,7 +68,7 @@ class CudaSolver(Solver):
         The call kernel's cells (wavefronts) per workgroup, stream batch, register budget in wavefronts per SIMD
         (1, or 2 for at most 256 registers with the excess spilled) and the rate coefficients' place (0: LDS, 1: a
         global scratch slot per wavefront); by default the autotuner's stored choice for this network and device,
-        else (1, 16, 1, 0).
+        else tune.default_variant's.
     tune : bool
         Run the autotuner now (maxichem_amd.tune) and store its choice.
     precision : str
