@@ -600,8 +600,25 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
   double c[NT];
   LeadRow a21;
   const int pairs = B * D;
-  while (q < pairs) {
-    const int dir = q / B, cell = q - dir * B;
+  // Where not every pair has a wavefront at once the queue passes over the pairs twice: first those whose first step is a small part of the call (dt > QUEUE_STEPS h:
+  // of settled cells about a tenth, among them every costly one), then the others. A launch lasts at least its costliest
+  // cell's tries, so that cell's pairs must not start late; skipping a pair costs about a microsecond of its wavefront. A
+  // cell's directions follow one another: they take the same tries (NCHO, settled cells by directions, in their order
+  // against this one: 1024 x 8 8.8 -> 7.9 ms, 4096 x 2 13.3 -> 11.8, 65,536 x 1 36.7 -> 31.9).
+  constexpr double QUEUE_STEPS = 12.0;
+  const int end = pairs > waves ? 2 * pairs : pairs;
+  auto take = [&] {
+    int nx = 0;
+    if (lane == 0) nx = waves + atomicAdd(count + COUNT_QUEUE, 1);
+    return __builtin_amdgcn_readfirstlane(nx);
+  };
+  auto skipped = [&](int i) {  // place i of the queue is a pair of its other pass
+    const int pass = i < pairs ? 0 : 1, at = (i - pass * pairs) / D;
+    return end > pairs && __builtin_amdgcn_readfirstlane(dta[at] > QUEUE_STEPS * hin_a[at] ? 0 : 1) != pass;
+  };
+  while (q < end && skipped(q)) q = take();
+  while (q < end) {
+    const int pair = q < pairs ? q : q - pairs, cell = pair / D, dir = pair - cell * D;
     const bool lead = dir == 0;  // direction 0's pair writes the call's results and counts
     const size_t dc = (size_t)dir * B + cell;  // the pair's row in the per-direction arrays
     const double Tc = Ta[cell], dt = dta[cell], nd = Pa[cell] / (KBOLTZ * Tc);
@@ -764,9 +781,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
       }
       redo[cell] = code != 0 ? 1 : 0;
     }
-    int nx = 0;
-    if (lane == 0) nx = waves + atomicAdd(count + COUNT_QUEUE, 1);
-    q = __builtin_amdgcn_readfirstlane(nx);
+    do q = take();
+    while (q < end && skipped(q));
   }
 }
 
@@ -827,7 +843,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   const bool ad = adapt != 0;
   int q = (int)blockIdx.x;
   while (q < pairs) {
-    const int dir = q / nfl, cell = list[q - dir * nfl];
+    const int at = q / D, dir = q - at * D, cell = list[at];
     const size_t dc = (size_t)dir * B + cell;  // the pair's row in the per-direction arrays
     const double Tc = Ta[cell], dt = dta[cell], nd = Pa[cell] / (KBOLTZ * Tc);
     const double* xr = x0 + (size_t)cell * NS;
