@@ -149,15 +149,15 @@ __device__ __forceinline__ void tie(float& a, float b) { asm volatile("" : "+v"(
 __device__ __forceinline__ bool wave_all(bool p) { return __ballot(!p) == 0ull; }
 
 // A stream word's term: d times the word's coefficient, exactly as fma(coefficient, d, .) takes it: x2 is an exponent
-// step, and the sign (the word's bit 31) is XORed into the double's sign bit, or put there where d is not SIGNED (then
-// one instruction). No compares and selects, and no wait states for condition masks.
+// step, and the sign (the word's bit 31) is XORed into the double's sign bit (one v_bitop3 with its mask; d may be
+// negative, a derivative too: an efficiency below 0 makes its reaction's rates negative). No compares and selects, and
+// no wait states for condition masks.
 static_assert(T_NEG == 31 && SV_NEG == 31, "the streams' sign bit is the word's sign bit");
-template <int DBL, bool SIGNED = true>
+template <int DBL>
 __device__ __forceinline__ double term(u32 w, double d) {
   d = __builtin_amdgcn_ldexp(d, (int)((w >> DBL) & 1u));
   const long long b = __double_as_longlong(d);
-  const u32 hi = (u32)((u64)b >> 32);
-  const u32 h = SIGNED ? hi ^ (w & 0x80000000u) : (hi & 0x7fffffffu) | (w & 0x80000000u);
+  const u32 h = (u32)((u64)b >> 32) ^ (w & 0x80000000u);
   return __longlong_as_double((long long)((u64)h << 32 | (u32)b));
 }
 
@@ -322,8 +322,7 @@ __device__ __forceinline__ void lds_add(double* p, double d) {
 // built). The last batch's words are loaded before the terms of the batch ahead of it are read, those of a stream of one
 // batch by its caller, so that it does not wait for them (NCHO, with the rates ahead in rhs: 256 cold cells
 // 17.3 -> 16.6 ms, 65,536 settled 7.5 -> 7.15 ms; the loop's words carried from batch to batch as well: no faster, and
-// the module takes 62 s to compile instead of 40). SIGNED: the terms may be negative; else the word's sign bit is put in
-// place of theirs.
+// the module takes 62 s to compile instead of 40).
 using StreamWords = u32[STREAM_BATCH];
 
 // The words of a stream's rounds from q0 on, at most a batch of them.
@@ -340,7 +339,7 @@ __device__ __forceinline__ void load_ahead(WP words, StreamWords& w, int lane) {
 }
 
 // w: what load_ahead loaded. next(w): called when the last batch's words are in use, to load another stream's ahead.
-template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, bool SIGNED, int ROUNDS, typename WP, typename Next>
+template <unsigned IDX_MASK, int DBL, int DEST, unsigned DEST_MASK, int ROUNDS, typename WP, typename Next>
 __device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const double* src, double* dst, int lane, Next next) {
   constexpr int LAST = ROUNDS > 0 ? (ROUNDS - 1) / STREAM_BATCH * STREAM_BATCH : 0;  // the last batch's first round
   auto batch = [&](StreamWords& from, int n, auto load) {  // n <= STREAM_BATCH rounds
@@ -355,7 +354,7 @@ __device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const doubl
 #pragma unroll
     for (int i = 0; i < STREAM_BATCH; i++) {
       if (i >= n) break;
-      lds_add(dst + ((cur[i] >> DEST) & DEST_MASK), term<DBL, SIGNED>(cur[i], d[i]));
+      lds_add(dst + ((cur[i] >> DEST) & DEST_MASK), term<DBL>(cur[i], d[i]));
     }
   };
 #pragma unroll 1
@@ -373,8 +372,7 @@ __device__ __forceinline__ void stream_sum(WP words, StreamWords& w, const doubl
 // One Jacobian stream into the cell's LDS: entries of -Jn at their offsets.
 template <int ROUNDS, typename WP, typename Next>
 __device__ __forceinline__ void jac_stream(WP words, StreamWords& w, const double* DV, double* ws, int lane, Next next) {
-  // dv terms are not negative
-  stream_sum<T_IDX_MASK, T_DBL, T_DEST, T_DEST_MASK, false, ROUNDS>(words, w, DV, ws, lane, next);
+  stream_sum<T_IDX_MASK, T_DBL, T_DEST, T_DEST_MASK, ROUNDS>(words, w, DV, ws, lane, next);
 }
 
 // The stream words in the workgroup's LDS (WORDS_LDS: the call kernel copies them there at its start, after its
@@ -464,7 +462,7 @@ __device__ __forceinline__ double rhs(double Yl, double Yt, double& Fl, double& 
     if (i + lane < NPART) part[i + lane] = 0.0;
   if (lane == 0) V[NR] = 0.0;  // the S v stream's padding term
   wave_sync();
-  stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, true, SV_ROUNDS>(svp, sw, V, part, lane, [](StreamWords&) {});
+  stream_sum<SV_R_MASK, SV_DBL, SV_PIECE, SV_PIECE_MASK, SV_ROUNDS>(svp, sw, V, part, lane, [](StreamWords&) {});
   wave_sync();
   // each row's pieces in order; the reads go out together (a row of fewer pieces than the most reads within part)
   auto row = [&](u32 rp) {
