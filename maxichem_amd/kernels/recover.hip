@@ -147,10 +147,24 @@ __device__ __forceinline__ bool dense_lu_2d(double* W, int* pr, double* dinv, do
   return true;
 }
 
+// A pointer into LDS, as a function that is called takes it.
+template <typename T>
+using lptr = __attribute__((address_space(3))) T*;
+
+// dense_lu_2d as a function of its own, in every network that has the register LU: the compiler then allocates its
+// registers apart from the tries' (which it keeps over the call, 1.0 KB a lane on NCHO, 2.2 KB on SNCHO). Inlined, the
+// recovery takes as long but SNCHO's spills 211 registers and its module takes 105 s to compile instead of 37 s (NCHO's
+// 20 s instead of 12 s). 500 cold cells, 40 tries each, ms: NCHO 29-36 here, 30-34 inlined, 54-56 by dense_lu alone; SNCHO,
+// the largest block (138 slots), 62-69, 64-74 and 88-90.
+__device__ __attribute__((noinline)) bool dense_lu_called(lptr<double> W, lptr<int> pr, lptr<double> dinv, lptr<double> lb,
+                                                          int lane) {
+  return dense_lu_2d((double*)W, (int*)pr, (double*)dinv, (double*)lb, lane);
+}
+
 // W's factors for the workgroup's first wavefront: in its registers, or with the other wavefronts (cmd calls them).
 __device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane) {
   if constexpr (LU_2D) {
-    if (dense_lu_2d(W, pr, dinv, ws + L_DV, lane)) return;
+    if (dense_lu_called((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane)) return;
   }
   if (lane == 0) *cmd = 1;
   __syncthreads();
