@@ -4,12 +4,14 @@ per SIMD) and the rate coefficients' place (LDS or global scratch), per network,
 Each candidate is compiled, loaded and timed by HIP events around the call kernel on a sample of the workload:
 "uneven", one synthetic call from cold (solar gas, dt log-uniform 1e1-1e4 s, half of the cells lit), or "settled",
 calls of dt = 300 s after a dark relaxation (the GPU FP64 case's sequence, a quarter of the cells lit). The fastest
-is stored in the code cache (tune.json) under the network's table digest, the photolysis switch, the device name and
-the workload, and later solvers of that network on that device take the uneven choice unless told the workload.
+is stored in the code cache (tune.json) under the network's table digest, the photolysis switch, the device name, the
+kernels it was timed on, the precision and the workload, and later solvers of that network on that device take the
+uneven choice unless told the workload.
 """
 
 from __future__ import annotations
 
+import hashlib
 import json
 import os
 from pathlib import Path
@@ -54,32 +56,41 @@ def _store() -> Path:
 WORKLOADS = ("uneven", "settled")
 
 
-def _key(net, photo: bool, device: torch.device, workload: str = "uneven") -> str:
-    key = f"{_tables.build(net, photo).digest()}|{int(photo)}|{torch.cuda.get_device_name(device)}"
-    return key if workload == "uneven" else f"{key}|{workload}"
+def kernels_digest() -> str:
+    """What a choice was timed on: the kernel files, the modules that write their header and tables, the compiler and its
+    options. A choice outlives none of them: other kernels have another best variant."""
+    files = [_kernels.KERNEL_DIR / name for name in (*_kernels.KERNEL_FILES, "mixed.hip")]
+    parts = [f.read_bytes() for f in (*files, Path(_kernels.__file__), Path(_tables.__file__))]
+    options = repr((_kernels.OPTIONS, _hip.compiler_version())).encode()
+    return hashlib.sha256(b"\0".join([*parts, options])).hexdigest()[:16]
 
 
-def stored(net, device, photo: bool, workload: str = "uneven") -> dict | None:
+def _key(net, photo: bool, device: torch.device, workload: str = "uneven", mixed: bool = False) -> str:
+    key = f"{_tables.build(net, photo).digest()}|{int(photo)}|{torch.cuda.get_device_name(device)}|{kernels_digest()}"
+    return key + ("|mixed" if mixed else "") + ("" if workload == "uneven" else f"|{workload}")
+
+
+def stored(net, device, photo: bool, workload: str = "uneven", mixed: bool = False) -> dict | None:
     try:
-        return json.loads(_store().read_text()).get(_key(net, photo, device, workload))
+        return json.loads(_store().read_text()).get(_key(net, photo, device, workload, mixed))
     except (OSError, ValueError):
         return None
 
 
 def choose(net, device, photo: bool, drift: float, run: bool = False, workload: str = "uneven",
            mixed: bool = False) -> tuple[int, ...]:  # fmt: skip
-    """The variant for this network, device and workload: tuned now when run, else the stored choice, else
-    default_variant."""
+    """The variant for this network, device, workload and form (FP64 or mixed): tuned now when run, else the stored
+    choice, else default_variant."""
     if run:
-        return tuple(tune(net, device, photo, drift, workload=workload)["best"])
-    s = stored(net, device, photo, workload)
+        return tuple(tune(net, device, photo, drift, workload=workload, mixed=mixed)["best"])
+    s = stored(net, device, photo, workload, mixed)
     return tuple(s["best"]) if s else default_variant(_tables.build(net, photo), mixed)
 
 
 def tune(net, device, photo: bool, drift: float, cells: int = 8192, seed: int = 7, repeats: int = 2,
-         workload: str = "uneven") -> dict:  # fmt: skip
-    """Time every variant on the workload's sample; store and return {"best", "ms": {variant: ms}, "private_bytes":
-    {variant: bytes per lane the variant spills}}."""
+         workload: str = "uneven", mixed: bool = False) -> dict:  # fmt: skip
+    """Time every variant of the FP64 or the mixed form on the workload's sample; store and return {"best", "ms":
+    {variant: ms}, "private_bytes": {variant: bytes per lane the variant spills}}."""
     from .kincuda import CudaSolver
 
     if workload not in WORKLOADS:
@@ -105,7 +116,7 @@ def tune(net, device, photo: bool, drift: float, cells: int = 8192, seed: int = 
             x, h, dtt = r.x, r.h, g(d["dt"])
     ms, spills = {}, {}
     for v in VARIANTS:
-        with CudaSolver(net, dev, photo=photo, drift=drift, variant=v) as s:
+        with CudaSolver(net, dev, photo=photo, drift=drift, variant=v, precision="mixed" if mixed else "fp64") as s:
             s(x, T, P, dtt, h, J=J)  # the first call pays for loading
             s.timing = []
             for _ in range(repeats):
@@ -123,7 +134,7 @@ def tune(net, device, photo: bool, drift: float, cells: int = 8192, seed: int = 
         data = json.loads(path.read_text()) if path.exists() else {}
     except ValueError:
         data = {}
-    data[_key(net, photo, dev, workload)] = out
+    data[_key(net, photo, dev, workload, mixed)] = out
     try:
         path.parent.mkdir(parents=True, exist_ok=True)
         tmp = path.with_suffix(f".tmp{os.getpid()}")
