@@ -240,19 +240,15 @@ def lds_bytes(tab: Tables, cpw: int, mixed: bool = False, rates_global: bool = F
 def every_destination(words: np.ndarray, end: int, dest: int, spare: np.ndarray) -> np.ndarray:
     """A stream's words [rounds, lanes] with the destination of the entry they belong to in every word (the tables hold
     it in the entry's last word, which keeps its mark). A lane's padding words take its last entry's, or spare[lane]."""
-    low = np.uint32((1 << dest) - 1)
-    field = np.uint32(0x7FFFFFFF) & ~low  # the destination's bits: from dest to the sign bit
-    out = words.copy()
-    for lane in range(words.shape[1]):
-        place = np.uint32(int(spare[lane]) << dest)
-        ends = np.flatnonzero(words[:, lane] >> np.uint32(end) & 1)
-        if len(ends):
-            place = words[ends[-1], lane] & field
-        for r in range(words.shape[0] - 1, -1, -1):
-            if words[r, lane] >> np.uint32(end) & 1:
-                place = words[r, lane] & field
-            out[r, lane] = (words[r, lane] & ~field) | place
-    return out
+    field = np.uint32(0x7FFFFFFF >> dest << dest)  # the destination's bits: from dest to the sign bit
+    rounds, lanes = words.shape
+    at = np.where(words >> np.uint32(end) & 1, np.arange(rounds)[:, None], -1)  # a round that ends an entry: its own
+    last = at.max(0, initial=-1)
+    ends = np.where(at < 0, rounds, at)
+    ends = np.minimum.accumulate(ends[::-1], 0)[::-1]  # else the lane's next one; past its last, that one
+    ends = np.where(ends < rounds, ends, last[None, :])
+    place = np.where(last < 0, spare.astype(np.uint32) << np.uint32(dest), words[ends, np.arange(lanes)] & field)
+    return (words & ~field) | place.astype(np.uint32)
 
 
 def host_tables(tab: Tables) -> dict[str, np.ndarray]:
