@@ -35,6 +35,12 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The places of a queue of pairs that is passed over twice where there are more pairs than wavefronts; once also where
+// two passes' places, and the one each wavefront takes past the end, would not fit an int.
+__device__ __forceinline__ int queue_places(int pairs, int waves) {
+  return pairs > waves && pairs <= (0x7fffffff - waves) / 2 ? 2 * pairs : pairs;
+}
+
 // Lane l's value of v, for a wave-uniform l (v_readlane, no LDS).
 __device__ __forceinline__ double readlane(double v, int l) {
   const long long b = __double_as_longlong(v);

@@ -600,13 +600,14 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
   double c[NT];
   LeadRow a21;
   const int pairs = B * D;
-  // Where not every pair has a wavefront at once the queue passes over the pairs twice: first those whose first step is a small part of the call (dt > QUEUE_STEPS h:
-  // of settled cells about a tenth, among them every costly one), then the others. A launch lasts at least its costliest
-  // cell's tries, so that cell's pairs must not start late; skipping a pair costs about a microsecond of its wavefront. A
-  // cell's directions follow one another: they take the same tries (NCHO, settled cells by directions, in their order
-  // against this one: 1024 x 8 8.8 -> 7.9 ms, 4096 x 2 13.3 -> 11.8, 65,536 x 1 36.7 -> 31.9).
+  // Where not every pair has a wavefront at once (queue_places) the queue passes over the pairs twice: first those whose
+  // first step is a small part of the call (dt > QUEUE_STEPS h: of settled cells about a tenth, among them every costly
+  // one), then the others. A launch lasts at least its costliest cell's tries, so that cell's pairs must not start late;
+  // skipping a pair costs about a microsecond of its wavefront. A cell's directions follow one another: they take the
+  // same tries (NCHO, settled cells by directions, in their order against this one: 1024 x 8 8.8 -> 7.9 ms, 4096 x 2
+  // 13.3 -> 11.8, 65,536 x 1 36.7 -> 31.9).
   constexpr double QUEUE_STEPS = 12.0;
-  const int end = pairs > waves ? 2 * pairs : pairs;
+  const int end = queue_places(pairs, waves);
   auto take = [&] {
     int nx = 0;
     if (lane == 0) nx = waves + atomicAdd(count + COUNT_QUEUE, 1);
