@@ -861,7 +861,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
     const double dtdc = (ad && dtd) ? dtd[dc] : 0.0;
     const double h0d = !ad ? 0.0 : (isfinite(hin[cell]) ? (hd ? hd[dc] : 0.0) : dtdc);
     const double md = h0 < dt ? h0d : (h0 > dt ? dtdc : 0.5 * (h0d + dtdc));  // m's tangent
-    int ntry = 0;
+    int ntry = 0, exchanged = 0;
     for (int pass = 0;; pass++) {
       const gptr<int> perm = opaque(net)->perm;
       double Nl = lane < K0 ? xr[perm[lane]] : 0.0, Nt = lane < NT ? xr[perm[K0 + lane]] : 0.0;
@@ -894,7 +894,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
           for (int j = 0; j < NT; j++) row[K0 + j] = (j == lane ? c[j] + igh : c[j]) - ut;
         }
         wave_sync();
-        dense_factor(W, pr, dinv, ws, cmd, lane);
+        dense_factor(W, pr, dinv, ws, cmd, lane, exchanged);
         double K1l, K1t, K2l, K2t, K3l, K3t, K4l, K4t;
         to_lds(yv, Fl, Ft, lane);
         dense_solve(W, pr, dinv, yv, lane);

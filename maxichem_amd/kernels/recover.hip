@@ -162,13 +162,29 @@ __device__ __attribute__((noinline)) bool dense_lu_called(lptr<double> W, lptr<i
 }
 
 // W's factors for the workgroup's first wavefront: in its registers, or with the other wavefronts (cmd calls them).
-__device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane) {
+// exchanged: the cell's last tries in a row whose W exchanged rows (0 at the cell's start). After DENSE_EXCHANGES of them the
+// registers are not tried until one exchanges none: two cells that exchange in nearly all of their 40,000 tries take 3.92 s,
+// with the registers tried first each time 4.46 s. Fewer would send a cell that exchanges now and then (6 % of the tries of
+// 367 recovered NCHO cells) to dense_lu, whose 162k cycles are five times the registers' 33k.
+constexpr int DENSE_EXCHANGES = 4;
+
+__device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane,
+                                             int& exchanged) {
   if constexpr (LU_2D) {
-    if (dense_lu_called((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane)) return;
+    if (exchanged < DENSE_EXCHANGES &&
+        dense_lu_called((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane)) {
+      exchanged = 0;
+      return;
+    }
   }
   if (lane == 0) *cmd = 1;
   __syncthreads();
   dense_lu(W, pr, dinv, lane, 0);
+  if constexpr (LU_2D) {
+    bool moved = false;
+    for (int i = lane; i < NS; i += WAVE) moved |= pr[i] != i;
+    exchanged = __ballot(moved) ? exchanged + 1 : 0;
+  }
 }
 
 // y <- W^-1 y with dense_lu's factors; y is the vector in LDS (elimination order). Up to ROW_REGISTERS species, this
@@ -294,7 +310,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
     cell_rates(ws, rk, Tc, nd, net, Jc, lane);
     const double h0 = isfinite(hin[cell]) ? hin[cell] : dt;
     const double m = fmin(h0, dt);
-    int ntry = 0;
+    int ntry = 0, exchanged = 0;
     for (int pass = 0;; pass++) {
       const gptr<int> perm = opaque(net)->perm;
       double Nl = lane < K0 ? xr[perm[lane]] : 0.0, Nt = lane < NT ? xr[perm[K0 + lane]] : 0.0;
@@ -320,7 +336,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
           for (int j = 0; j < NT; j++) row[K0 + j] = (j == lane ? c[j] + igh : c[j]) - ut;
         }
         wave_sync();
-        dense_factor(W, pr, dinv, ws, cmd, lane);
+        dense_factor(W, pr, dinv, ws, cmd, lane, exchanged);
         double K1l, K1t, K2l, K2t, K3l, K3t, K4l, K4t;
         to_lds(yv, Fl, Ft, lane);
         dense_solve(W, pr, dinv, yv, lane);
