@@ -342,7 +342,7 @@ def run_learned(args, net, dev) -> int:
         return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
 
     x, T, P, dt, h, J = (g(d[k]) for k in ("x", "T", "P", "dt", "h", "J"))
-    plain = CudaSolver(net, dev, photo=True, variant=(1, 16, 1, 0))
+    plain = CudaSolver(net, dev, photo=True)  # the variant the learned solvers take too
     t0 = time.perf_counter()
     data = generate(plain, learned_training_sequences(net, args.train_pairs, args.train_cells))
     npairs = int(data["x0"].shape[0])
