@@ -33,7 +33,7 @@ FP64_PEAK = 78.6  # TFLOP/s, MI355X FP64 vector
 # HBM bytes the plain FP64 call kernel (its guard included) moves per cell-call on the 69-species workload: a constant
 # from the FETCH_SIZE and WRITE_SIZE counters of separate profiled runs of this bench (timed calls), scaled by what
 # they read for a 512 MiB copy (x2 and x1), profiles/mxc_call_ncho_65536_traffic.md; not measured in this run
-TRAFFIC_PER_CELL_CALL = {"NCHO": 2048}
+TRAFFIC_PER_CELL_CALL = {"NCHO": 20200}
 HEADLINE_MARGIN = 1.02  # another form heads the line only when it beats the plain one by more than this
 TRAFFIC_SOURCE = "profiles/mxc_call_ncho_65536_traffic.md (rocprofv3 FETCH_SIZE, WRITE_SIZE; a constant, not this run)"
 

@@ -101,7 +101,10 @@ def words_in_lds(tab: Tables, cpw: int, mixed: bool = False, wps: int = 1, rates
 
 # The two-dimensional LU up to here: its block takes 180 registers at 69 species and 276 at 92, which a wavefront alone
 # on its SIMD holds (256, and accumulation registers for what rests); 128 species would take 512. Larger networks keep
-# the LU by rows.
+# the LU by rows. The line is where the largest block was that had been timed; beyond it the LU by rows is slower still
+# (4,096 cold cells, settled ones, 256 recovered ones, ms by rows and with the line raised: 93 species 77.4 and 30.3, 22.9
+# and 8.9, 52.5 and 36; 110 species 264 and 62.8, 43 and 10.5, 73.9 and 52.6) and quicker to compile (a call and a tangent
+# module of 93 species 63 s in registers).
 LU_MAX_SPECIES = 92
 
 

@@ -922,8 +922,9 @@ __device__ __forceinline__ bool lu_inside(int m, int t, int lane) {
   return (i + 16 <= ni || i + (lane & 15) < ni) && (j + 4 <= nj || j + (lane >> 4) < nj);
 }
 
-// A from the rows by lane (c, a21, and the lead rows in LDS; a caller that has the matrix by rows): columns pass LU_CHUNK slots at a time through the cell's
-// LDS from its dv terms on, which no later part of a try reads.
+// A from the rows by lane (c, a21, and the lead rows in LDS), for a caller that has the matrix by rows, as the LU's tests
+// do (a try assembles straight into the slots, lu_assemble): columns pass LU_CHUNK slots at a time through the cell's LDS
+// from its dv terms on, which no later part of a try reads.
 __device__ __forceinline__ void lu_load(LuBlock& A, const double (&c)[NT], const LeadRow& a21, double* ws, int lane) {
   const LuPlace p(ws, lane);
   double* buf = ws + L_DV;

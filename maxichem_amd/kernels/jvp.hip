@@ -605,7 +605,11 @@ extern "C" __global__ void __launch_bounds__(WAVE* CPW)
   // one), then the others. A launch lasts at least its costliest cell's tries, so that cell's pairs must not start late;
   // skipping a pair costs about a microsecond of its wavefront. A cell's directions follow one another: they take the
   // same tries (NCHO, settled cells by directions, in their order against this one: 1024 x 8 8.8 -> 7.9 ms, 4096 x 2
-  // 13.3 -> 11.8, 65,536 x 1 36.7 -> 31.9).
+  // 13.3 -> 11.8, 65,536 x 1 36.7 -> 31.9). The line of 12 is from settled cells of dt = 300 s, where the second pass by
+  // itself takes 16,384 x 1 pairs from 14.9 to 13.4 ms or leaves them at 13.9, as the costliest cell falls. Elsewhere, one
+  // pass against two, 4096 x 2: settled cells of dt = 3,000 s (a quarter of them first) 34.6 -> 33.8 ms; where all come
+  // first (dt = 1e6 s, cold cells) the same; where none does (dt = 10 s, 1.1 tries each) 1.89 -> 1.97 ms, the price of
+  // passing over every pair.
   constexpr double QUEUE_STEPS = 12.0;
   const int end = queue_places(pairs, waves);
   auto take = [&] {

@@ -54,7 +54,8 @@ class LaunchResult(NamedTuple):
 
 
 class CudaSolver(Solver):
-    """Batched chemistry solver on one GPU; calls run one at a time on torch's current stream.
+    """Batched chemistry solver on one GPU; calls run one at a time on torch's current stream (they share the counts, the
+    queues and, with rates in global scratch, the slots of rate coefficients).
 
     Parameters
     ----------
@@ -285,9 +286,11 @@ class CallGraph:
     """One call of a solver captured in a HIP graph on fixed tensors (a GCM's time loop calls with the same tensors
     every step): replay() runs the call kernel (with its guard) and the recovery again on what the input tensors
     hold then, with one launch, and returns the graph's own output tensors, which the next replay overwrites. The
-    graph owns every buffer its kernels address, the mixed form's FP64 flags included. The counts, the
-    refusals and check() behave as in an eager call; the queue is ordered by the previous replay's tries, set on the
-    host side before each replay. Building it runs the call once, off the graph, without adding to the counts."""
+    graph owns its outputs, its queue's order and the mixed form's FP64 flags; it shares the solver's tables, counts and,
+    where the rate coefficients are in global scratch (NCHO's default), their slots, so a replay must not overlap another
+    call of its solver. The counts, the refusals and check() behave as in an eager call; the queue is ordered by the
+    previous replay's tries, set on the host side before each replay. Building it runs the call once, off the graph,
+    without adding to the counts."""
 
     def __init__(self, solver: CudaSolver, x, T, P, dt, h, *, rtol: float = DEFAULT_RTOL, atol: float = ATOL,
                  max_steps: int = DEFAULT_MAX_STEPS, J=None) -> None:  # fmt: skip

@@ -234,7 +234,7 @@ class ADSolver(CudaSolver):
     def _column_chunks(self, columns: int, B: int):
         """The vjp's columns [first, last) of each launch: as many directions as their unit tangents and outputs take
         COLUMN_BYTES. A launch lasts at least its costliest cell's tries and a host visit costs about 0.1 ms, so fewer,
-        fuller launches (64 NCHO cells, 509 columns: 41 ms in eight launches with a recovery launch per column, 13.5 ms
+        fuller launches (64 NCHO cells, 511 columns: 41 ms in eight launches with a recovery launch per column, 13.5 ms
         in one)."""
         per = 8 * B * (2 * self.ns + 4 + self.nj + self.nr)  # one direction's tangents and outputs, at most
         size = max(1, min(COLUMN_BYTES // max(per, 1), columns))

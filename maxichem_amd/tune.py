@@ -31,9 +31,10 @@ CU_WAVES = 4  # call wavefronts per compute unit at one per SIMD
 def default_variant(tab, mixed: bool = False) -> tuple[int, int, int, int]:
     """The variant without a stored choice, with the same bits as every other. Two wavefronts per SIMD where a compute
     unit's LDS holds eight cells (with the rates in LDS, else in global scratch): each waits for its LDS reads and
-    chains of broadcasts while the other issues, which outweighs the few registers it spills (NCHO, kernel ms: 8,192
-    cold cells 45.2 -> 32.4, 65,536 settled cells 12.5 -> 12.0, 256 cold cells 20.4 -> 18.7). Else, and in the mixed
-    form: four cells per workgroup when the stream words then fit in the workgroup's LDS at as many cells per compute
+    chains of broadcasts while the other issues, which outweighs the few registers it spills (NCHO, ms a call against
+    (4, 16, 1, 0), two draws each: 65,536 settled cells 11.5 -> 7.2 and 11.6 -> 11.1, 256 cold cells 18.7 -> 16.5 and
+    22.0 -> 19.9, 8,192 cold cells 41.0 -> 28.9 and, where one cell's 1,439 tries are the call, 51.5 -> 52.3). Else, and
+    in the mixed form: four cells per workgroup when the stream words then fit in the workgroup's LDS at as many cells per compute
     unit; else two when that keeps as many cells per compute unit as one; else one."""
     if not mixed and _kernels.lu_layout(tab)["use"]:
         for rates_global in (0, 1):
