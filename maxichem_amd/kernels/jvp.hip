@@ -837,11 +837,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(yv + NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    for (;;) {
-      __syncthreads();
-      if (*cmd == 0) return;
-      dense_lu(W, pr, dinv, lane, wv);
-    }
+    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane, wv);
+    return;
   }
   double c[NT];
   LeadRow a21;
@@ -1021,7 +1018,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
       break;
     }
   }
-  if (lane == 0) *cmd = 0;
+  if (lane == 0) *cmd = DENSE_END;
   __syncthreads();  // the other wavefronts leave
 }
 

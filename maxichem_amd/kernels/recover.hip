@@ -147,37 +147,65 @@ __device__ __forceinline__ bool dense_lu_2d(double* W, int* pr, double* dinv, do
   return true;
 }
 
+// A recovery workgroup's factorizations. Its first wavefront steps the cell and asks for them through a word in LDS (cmd);
+// the others wait for it at a workgroup barrier.
+constexpr int DENSE_END = 0, DENSE_ALL = 1, DENSE_REGISTERS = 2;  // cmd: leave; factor W together; the second alone
+
 // A pointer into LDS, as a function that is called takes it.
 template <typename T>
 using lptr = __attribute__((address_space(3))) T*;
 
-// dense_lu_2d as a function of its own, in every network that has the register LU: the compiler then allocates its
-// registers apart from the tries' (which it keeps over the call, 1.0 KB a lane on NCHO, 2.2 KB on SNCHO). Inlined, the
-// recovery takes as long but SNCHO's spills 211 registers and its module takes 105 s to compile instead of 37 s (NCHO's
-// 20 s instead of 12 s). 500 cold cells, 40 tries each, ms: NCHO 29-36 here, 30-34 inlined, 54-56 by dense_lu alone; SNCHO,
-// the largest block (138 slots), 62-69, 64-74 and 88-90.
-__device__ __attribute__((noinline)) bool dense_lu_called(lptr<double> W, lptr<int> pr, lptr<double> dinv, lptr<double> lb,
-                                                          int lane) {
-  return dense_lu_2d((double*)W, (int*)pr, (double*)dinv, (double*)lb, lane);
+// What the other wavefronts do until the workgroup's cells are done, as a function of its own that they enter once. The LU in
+// registers runs here, in the second wavefront, while the first waits: no register of a try is held or saved around its
+// block, and the compiler allocates the two apart. 500 cold cells of 40 tries each, ms: NCHO 28-34, SNCHO (the largest
+// block, 138 slots) 56-68, by dense_lu alone 54-56 and 88-90. Inlined into the tries it was no faster (29-36 and 61-75),
+// spilled 211 registers on SNCHO and took its module 105 s to compile instead of 43 s (NCHO's 20 s instead of 14 s); called
+// from each try it kept 1.0 KB a lane over the call (SNCHO 2.2 KB) and took 2 % longer.
+__device__ __attribute__((noinline)) void dense_workers(lptr<double> Wl, lptr<int> prl, lptr<double> dinvl, lptr<double> lbl,
+                                                        int lane, int wv) {
+  double *W = (double*)Wl, *dinv = (double*)dinvl, *lb = (double*)lbl;
+  int* pr = (int*)prl;
+  volatile int* cmd = pr + NS;
+  wv = __builtin_amdgcn_readfirstlane(wv);
+  for (;;) {
+    __syncthreads();
+    const int what = __builtin_amdgcn_readfirstlane(*cmd);
+    if (what == DENSE_END) return;
+    if constexpr (LU_2D) {
+      if (what == DENSE_REGISTERS) {
+        if (wv == 1) dense_lu_2d(W, pr, dinv, lb, lane);
+        __syncthreads();
+        continue;
+      }
+    }
+    dense_lu(W, pr, dinv, lane, wv);
+  }
 }
 
-// W's factors for the workgroup's first wavefront: in its registers, or with the other wavefronts (cmd calls them).
-// exchanged: the cell's last tries in a row whose W exchanged rows (0 at the cell's start). After DENSE_EXCHANGES of them the
-// registers are not tried until one exchanges none: two cells that exchange in nearly all of their 40,000 tries take 3.92 s,
-// with the registers tried first each time 4.46 s. Fewer would send a cell that exchanges now and then (6 % of the tries of
-// 367 recovered NCHO cells) to dense_lu, whose 162k cycles are five times the registers' 33k.
+// W's factors, for the first wavefront. exchanged: the cell's last tries in a row whose W exchanged rows (0 at the cell's
+// start). After DENSE_EXCHANGES of them the registers are not tried until one exchanges none: two cells that exchange in
+// nearly all of their 40,000 tries take 3.85 s, with the registers tried first each time 4.45 s. Fewer would send a cell
+// that exchanges now and then (6 % of the tries of 367 recovered NCHO cells) to dense_lu, whose 162k cycles are five
+// times the registers' 33k.
 constexpr int DENSE_EXCHANGES = 4;
 
 __device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane,
                                              int& exchanged) {
   if constexpr (LU_2D) {
-    if (exchanged < DENSE_EXCHANGES &&
-        dense_lu_called((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane)) {
-      exchanged = 0;
-      return;
+    if (exchanged < DENSE_EXCHANGES) {
+      if (lane == 0) {
+        *cmd = DENSE_REGISTERS;
+        pr[0] = -1;  // the row order is written where the registers have the factors
+      }
+      __syncthreads();
+      __syncthreads();  // the second wavefront has them, or has left W as it was
+      if (__builtin_amdgcn_readfirstlane(pr[0]) == 0) {
+        exchanged = 0;
+        return;
+      }
     }
   }
-  if (lane == 0) *cmd = 1;
+  if (lane == 0) *cmd = DENSE_ALL;
   __syncthreads();
   dense_lu(W, pr, dinv, lane, 0);
   if constexpr (LU_2D) {
@@ -267,8 +295,7 @@ __device__ __forceinline__ void from_lds(const double* y, double& vl, double& vt
 }
 
 // A workgroup of REC_WAVES wavefronts per listed cell: wavefront 0 steps the cell; the others wait at a workgroup
-// barrier for each of its dense factorizations (cmd 1: factor W, 0: the workgroup's cells are done), so every
-// wavefront passes the same barriers.
+// barrier for each of its dense factorizations (dense_workers), so every wavefront passes the same barriers.
 extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
     mxc_recover(NetP __restrict__ net, const double* __restrict__ x0, const double* __restrict__ Ta,
                 const double* __restrict__ Pa, const double* __restrict__ dta, const double* __restrict__ hin,
@@ -292,11 +319,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(yv + NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    for (;;) {
-      __syncthreads();
-      if (*cmd == 0) return;
-      dense_lu(W, pr, dinv, lane, wv);
-    }
+    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane, wv);
+    return;
   }
   double c[NT];
   LeadRow a21;
@@ -390,6 +414,6 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
       break;
     }
   }
-  if (lane == 0) *cmd = 0;
+  if (lane == 0) *cmd = DENSE_END;
   __syncthreads();  // the other wavefronts leave
 }

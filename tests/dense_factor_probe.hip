@@ -12,11 +12,8 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(dinv + 2 * NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    for (;;) {
-      __syncthreads();
-      if (*cmd == 0) return;
-      dense_lu(W, pr, dinv, lane, wv);
-    }
+    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(lds + L_DV), lane, wv);
+    return;
   }
   int exchanged = 0;
   for (int b = 0; b < count; b++) {
@@ -34,6 +31,6 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
     for (int i = lane; i < NS; i += WAVE) rows[(size_t)b * NS + i] = pr[i];
     wave_sync();
   }
-  if (lane == 0) *cmd = 0;
+  if (lane == 0) *cmd = DENSE_END;
   __syncthreads();
 }

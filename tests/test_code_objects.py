@@ -1,5 +1,5 @@
-"""The recovery kernel's code object: the register LU is a function of its own, so the tries' registers are not spilled
-around its block (inlined, SNCHO's recovery spills 211 registers and takes the compiler a minute more; CPU)."""
+"""The recovery kernel's code object: the register LU is apart from the tries, so their registers are not spilled around its
+block (inlined into them, SNCHO's recovery spills 211 registers and takes the compiler a minute more; CPU)."""
 
 import re
 import subprocess
