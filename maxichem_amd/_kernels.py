@@ -108,6 +108,14 @@ def words_in_lds(tab: Tables, cpw: int, mixed: bool = False, wps: int = 1, rates
 LU_MAX_SPECIES = 92
 
 
+# The recovery's LU in registers up to so many slots (95: 73 to 76 species; NCHO's 69 take 90). There every slot is taken, and
+# with 100 slots (80 species) the recovery kernel spills. A kernel that spills needs scratch memory, which the runtime sets
+# aside for the whole device, per queue, at the first launch, empty ones too: with SNCHO's 138 slots in registers 430 MB to
+# 1.1 GB, also in a call that may not allocate (mxc_solver_call_static), and its module took 105 s to compile instead of 24
+# s. In registers its 500 cold cells of 40 tries took 57-75 ms, by the wavefronts' LU 88-90; NCHO's 28-36 and 54-57.
+LU_DENSE_SLOTS = 96
+
+
 def lu_layout(tab: Tables) -> dict:
     """The two-dimensional LU's layout (kernels/common.hip, factor_2d): register slots of 16 rows (m) by 4 columns
     (t), the lead rows' and columns' (ml, tl) first; per pivot, the row slots that hold an entry below it in its column
@@ -134,7 +142,8 @@ def lu_layout(tab: Tables) -> dict:
         stride, plain = stride + 16, wide
     need = max(64 * m, 16 * m + 4 * tl + C.WAVE)  # the multipliers' exchange; the diagonal and its reciprocals
     fits = plain > 0 and room >= need and 16 * ml * ns <= lay["SPARE"] + C.WAVE  # whole slots of lead rows are read
-    return {"use": ns <= LU_MAX_SPECIES and fits, "m": m, "t": t, "ml": ml, "tl": tl,
+    use = ns <= LU_MAX_SPECIES and fits
+    return {"use": use, "dense": use and m * t <= LU_DENSE_SLOTS, "m": m, "t": t, "ml": ml, "tl": tl,
             "rows": rows, "cols": cols, "live": live, "chunk": max(plain, 1), "stride": stride}  # fmt: skip
 
 
@@ -193,6 +202,7 @@ def header(tab: Tables, cpw: int, drift: float, batch: int = DEFAULT_BATCH, mixe
         f"__device__ constexpr unsigned long long TRAIL_FILL[{tab.nt}] = "
         f"{{{', '.join(f'{m}ull' for m in tab.trail_fill)}}};",
         f"constexpr bool LU_2D = {'true' if lu['use'] else 'false'};",
+        f"constexpr bool LU_DENSE = {'true' if lu['dense'] else 'false'};  // in the recovery",
         *(f"__device__ constexpr unsigned {name}[{len(lu[key])}] = {{{', '.join(f'{v}u' for v in lu[key])}}};"
           for name, key in (("LU_ROWS", "rows"), ("LU_COLS", "cols"), ("LU_LIVE", "live"))),
         f"#define HAS_TROE {int(tab.has_troe)}",

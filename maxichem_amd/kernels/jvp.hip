@@ -837,7 +837,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(yv + NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane, wv);
+    dense_workers(W, pr, dinv, ws + L_DV, cmd, lane, wv);
     return;
   }
   double c[NT];

@@ -151,27 +151,17 @@ __device__ __forceinline__ bool dense_lu_2d(double* W, int* pr, double* dinv, do
 // the others wait for it at a workgroup barrier.
 constexpr int DENSE_END = 0, DENSE_ALL = 1, DENSE_REGISTERS = 2;  // cmd: leave; factor W together; the second alone
 
-// A pointer into LDS, as a function that is called takes it.
-template <typename T>
-using lptr = __attribute__((address_space(3))) T*;
-
-// What the other wavefronts do until the workgroup's cells are done, as a function of its own that they enter once. The LU in
-// registers runs here, in the second wavefront, while the first waits: no register of a try is held or saved around its
-// block, and the compiler allocates the two apart. 500 cold cells of 40 tries each, ms: NCHO 28-34, SNCHO (the largest
-// block, 138 slots) 56-68, by dense_lu alone 54-56 and 88-90. Inlined into the tries it was no faster (29-36 and 61-75),
-// spilled 211 registers on SNCHO and took its module 105 s to compile instead of 43 s (NCHO's 20 s instead of 14 s); called
-// from each try it kept 1.0 KB a lane over the call (SNCHO 2.2 KB) and took 2 % longer.
-__device__ __attribute__((noinline)) void dense_workers(lptr<double> Wl, lptr<int> prl, lptr<double> dinvl, lptr<double> lbl,
-                                                        int lane, int wv) {
-  double *W = (double*)Wl, *dinv = (double*)dinvl, *lb = (double*)lbl;
-  int* pr = (int*)prl;
-  volatile int* cmd = pr + NS;
+// What the other wavefronts do until the workgroup's cells are done. The LU in registers (LU_DENSE) runs here, in the second
+// wavefront, while the first waits: no register of a try is held around its block, and the kernel needs no scratch memory.
+// (As a function called from each try it cost 1.0 KB of it a lane, 530 MB of the device, and 2 % of a recovery's time.)
+__device__ __forceinline__ void dense_workers(double* W, int* pr, double* dinv, double* lb, volatile int* cmd, int lane,
+                                              int wv) {
   wv = __builtin_amdgcn_readfirstlane(wv);
   for (;;) {
     __syncthreads();
     const int what = __builtin_amdgcn_readfirstlane(*cmd);
     if (what == DENSE_END) return;
-    if constexpr (LU_2D) {
+    if constexpr (LU_DENSE) {
       if (what == DENSE_REGISTERS) {
         if (wv == 1) dense_lu_2d(W, pr, dinv, lb, lane);
         __syncthreads();
@@ -184,14 +174,14 @@ __device__ __attribute__((noinline)) void dense_workers(lptr<double> Wl, lptr<in
 
 // W's factors, for the first wavefront. exchanged: the cell's last tries in a row whose W exchanged rows (0 at the cell's
 // start). After DENSE_EXCHANGES of them the registers are not tried until one exchanges none: two cells that exchange in
-// nearly all of their 40,000 tries take 3.85 s, with the registers tried first each time 4.45 s. Fewer would send a cell
+// nearly all of their 40,000 tries take 3.86 s, with the registers tried first each time 4.46 s. Fewer would send a cell
 // that exchanges now and then (6 % of the tries of 367 recovered NCHO cells) to dense_lu, whose 162k cycles are five
 // times the registers' 33k.
 constexpr int DENSE_EXCHANGES = 4;
 
 __device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, double* ws, volatile int* cmd, int lane,
                                              int& exchanged) {
-  if constexpr (LU_2D) {
+  if constexpr (LU_DENSE) {
     if (exchanged < DENSE_EXCHANGES) {
       if (lane == 0) {
         *cmd = DENSE_REGISTERS;
@@ -208,7 +198,7 @@ __device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, d
   if (lane == 0) *cmd = DENSE_ALL;
   __syncthreads();
   dense_lu(W, pr, dinv, lane, 0);
-  if constexpr (LU_2D) {
+  if constexpr (LU_DENSE) {
     bool moved = false;
     for (int i = lane; i < NS; i += WAVE) moved |= pr[i] != i;
     exchanged = __ballot(moved) ? exchanged + 1 : 0;
@@ -223,6 +213,8 @@ __device__ __forceinline__ void dense_factor(double* W, int* pr, double* dinv, d
 constexpr int ROW_REGISTERS = 80;
 constexpr bool ROW_IN_REGISTERS = NS <= ROW_REGISTERS;
 constexpr int DENSE_BATCH = 16;  // steps whose entries of a lane's second row are read together
+// Where a lane's row is not in registers its reads stay in their batch: all of them ahead took registers that the function
+// must save, and a kernel with saved registers needs scratch memory.
 
 __device__ void dense_solve(const double* W, const int* pr, const double* dinv, double* y, int lane) {
   double a[2];
@@ -244,6 +236,7 @@ __device__ void dense_solve(const double* W, const int* pr, const double* dinv, 
 #pragma unroll
   for (int k0 = 0; k0 < NS - 1; k0 += DENSE_BATCH) {
     double w1[DENSE_BATCH];
+    if (!ROW_IN_REGISTERS) __builtin_amdgcn_sched_barrier(0);
     second(w1, k0, 1);
 #pragma unroll
     for (int i = 0; i < DENSE_BATCH; i++) {
@@ -261,6 +254,7 @@ __device__ void dense_solve(const double* W, const int* pr, const double* dinv, 
 #pragma unroll
   for (int k1 = NS - 1; k1 > 0; k1 -= DENSE_BATCH) {
     double w1[DENSE_BATCH];
+    if (!ROW_IN_REGISTERS) __builtin_amdgcn_sched_barrier(0);
     second(w1, k1, -1);
 #pragma unroll
     for (int i = 0; i < DENSE_BATCH; i++) {
@@ -319,7 +313,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(yv + NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(ws + L_DV), lane, wv);
+    dense_workers(W, pr, dinv, ws + L_DV, cmd, lane, wv);
     return;
   }
   double c[NT];

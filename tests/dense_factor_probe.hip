@@ -12,7 +12,7 @@ extern "C" __global__ void __launch_bounds__(WAVE* REC_WAVES)
   int* pr = (int*)(dinv + 2 * NS);
   volatile int* cmd = pr + NS;
   if (wv != 0) {
-    dense_workers((lptr<double>)W, (lptr<int>)pr, (lptr<double>)dinv, (lptr<double>)(lds + L_DV), lane, wv);
+    dense_workers(W, pr, dinv, lds + L_DV, cmd, lane, wv);
     return;
   }
   int exchanged = 0;
