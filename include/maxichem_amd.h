@@ -119,7 +119,9 @@ int mxc_solver_call(mxc_solver* solver, void* stream, int cells, const double* x
  * more than MXC_STATIC_CELLS cells are refused (return 1, mxc_last_error says so) before any device work. Every
  * call of this entry point on one device shares that array, so such calls must not overlap on a device (one stream,
  * or synchronized between streams), whichever solver they use. No counterpart in the reference: it is for callers
- * that cannot allocate device memory in their call path (tight serving loops, allocation-free harnesses). */
+ * that cannot allocate device memory in their call path (tight serving loops, allocation-free harnesses). The runtime
+ * itself sets scratch memory aside at a kernel's first launch on a queue where the kernel spills: export a variant whose
+ * kernels do not ((1, 16, 1, 0), the default of export_network). */
 int mxc_solver_call_static(mxc_solver* solver, void* stream, int cells, const double* x, const double* T,
                            const double* P, const double* dt, const double* h, const double* J, double rtol,
                            double atol, int max_steps, double* x_out, double* h_out, int* done, double* steps,
